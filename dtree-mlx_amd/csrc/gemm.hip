@@ -33,6 +33,7 @@
 //     weights with the activation pair (two bf16 MFMAs) and q4 dequantises to
 //     bf16.
 #include "common.h"
+#include "gemm_long.h"
 
 namespace dtree {
 
@@ -1811,27 +1812,24 @@ static void launch_dp_any(const GemmParams& p, int epi, bool q4, bool h16, hipSt
   else lo ? launch_dp<true, KS, false>(p, epi, st) : launch_dp<false, KS, false>(p, epi, st);
 }
 
-// ---- long-M GEMM (prompt prefill): rows a multiple of 128 --------------------
+// ---- long-M GEMM (prompt prefill), q4 weights: rows a multiple of 128 --------
 // Compute-bound: a workgroup owns a 128-row x 128-column output tile over the
-// whole K. Per 64-wide K block the workgroup stages the tile's activation
-// blocks (4 row blocks, hi and lo planes) and weight blocks (4 column blocks)
-// in LDS, 16 bytes per thread per 4 KB block, double-buffered with one barrier
-// per K block (the next block's loads are in flight during the current
-// block's MFMAs). Wave w computes rows 64 (w / 2) .. + 63 x columns
-// 64 (w % 2) .. + 63 as 2 x 2 MFMA 32 x 32 tiles: 32 MFMAs per K block with
-// both planes. The finished tile goes through LDS to the same epilogues as
-// the skinny GEMMs, applied to 128 rows.
+// whole K. A K block (64) is one quantisation group; per block the workgroup
+// stages the tile's activation blocks (4 row blocks, hi and lo planes), 1 KB
+// of nibbles and 32 (scale, bias) words per 32-column block in LDS,
+// double-buffered with one barrier per K block (the next block's loads are in
+// flight during the current block's MFMAs). Wave w computes rows 64 (w / 2) ..
+// + 63 x columns 64 (w % 2) .. + 63 as 2 x 2 MFMA 32 x 32 tiles: each takes a
+// fresh MFMA sum of x (128 + q) per group and folds it in as acc += s * sum +
+// (b - 128 s) * sum(x), with sum(x) per row block from an MFMA of the staged
+// activations against bf16 ones. The finished tile goes through LDS to the
+// same epilogues as the skinny GEMMs, applied to 128 rows.
 constexpr int kLongRows = 128, kLongCols = 128;
 
-// Q4: group-64 q4 weights (DTREE_W_Q4G64). A K block is one quantisation
-// group: per 32-column block 1 KB of nibbles and 32 (scale, bias) words are
-// staged; each wave's 32 x 32 tiles take a fresh MFMA sum of x (128 + q) per
-// group and fold it in as acc += s * sum + (b - 128 s) * sum(x), with sum(x)
-// per row block from an MFMA of the staged activations against bf16 ones.
-template <bool LO, int EPI, bool Q4, bool H = false>
-__device__ __forceinline__ void long_gemm_body(const GemmParams& p) {
+template <bool LO, int EPI>
+__global__ __launch_bounds__(kThreads) void longq_gemm_kernel(GemmParams p) {
   constexpr int NPL = LO ? 2 : 1, ABLK = 4 * NPL;
-  constexpr int WBYTES = Q4 ? 4 * 1024 + 4 * 128 : 4 * 4096;            // weight bytes per stage
+  constexpr int WBYTES = 4 * 1024 + 4 * 128;                            // weight bytes per stage
   constexpr int STAGE = ABLK * 4096 + WBYTES;                           // bytes per stage
   constexpr int SMEM = 2 * STAGE > kLongRows * kLongCols * 4 ? 2 * STAGE : kLongRows * kLongCols * 4;
   __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM];
@@ -1852,10 +1850,9 @@ __device__ __forceinline__ void long_gemm_body(const GemmParams& p) {
     }
     rs[t] = r;
   }
-  // Staged per thread: ABLK activation pieces, then the weight pieces (bf16:
-  // 4 x 16 bytes; q4: 16 bytes of nibbles, and for t < 32 16 bytes of
-  // scale / bias words).
-  constexpr int NW = Q4 ? 2 : 4;
+  // Staged per thread: ABLK activation pieces, then 16 bytes of nibbles, and
+  // for t < 32 16 bytes of scale / bias words.
+  constexpr int NW = 2;
   u32x4_t ld[ABLK + NW];
   const uint32_t* wsb = reinterpret_cast<const uint32_t*>(p.w_sb);
   auto load_stage = [&](int kb) {
@@ -1865,35 +1862,23 @@ __device__ __forceinline__ void long_gemm_body(const GemmParams& p) {
       ld[rb * NPL] = ld_u32x4(p.x + blk);
       if (LO) ld[rb * NPL + NPL - 1] = ld_u32x4(p.x_lo + blk);
     }
-    if constexpr (Q4) {
-      const int cb = nt * 4 + (t >> 6);  // this thread's 32-column block
-      ld[ABLK] = cb * 32 < p.n ? ld_u32x4(reinterpret_cast<const uint32_t*>(p.w) + ((size_t)cb * nkb + kb) * 256 +
-                                          4 * (t & 63))
-                               : u32x4_t{0u, 0u, 0u, 0u};
-      if (t < 32) {
-        const int sbb = nt * 4 + (t >> 3);
-        ld[ABLK + 1] = sbb * 32 < p.n ? ld_u32x4(wsb + ((size_t)sbb * nkb + kb) * 32 + 4 * (t & 7))
-                                      : u32x4_t{0u, 0u, 0u, 0u};
-      }
-    } else {
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb)
-        ld[ABLK + cb] = (nt * 4 + cb) * 32 < p.n ? ld_u32x4(p.w + ((size_t)(nt * 4 + cb) * nkb + kb) * 2048 + 8 * t)
-                                                 : u32x4_t{0u, 0u, 0u, 0u};
+    const int cb = nt * 4 + (t >> 6);  // this thread's 32-column block
+    ld[ABLK] = cb * 32 < p.n ? ld_u32x4(reinterpret_cast<const uint32_t*>(p.w) + ((size_t)cb * nkb + kb) * 256 +
+                                        4 * (t & 63))
+                             : u32x4_t{0u, 0u, 0u, 0u};
+    if (t < 32) {
+      const int sbb = nt * 4 + (t >> 3);
+      ld[ABLK + 1] = sbb * 32 < p.n ? ld_u32x4(wsb + ((size_t)sbb * nkb + kb) * 32 + 4 * (t & 7))
+                                    : u32x4_t{0u, 0u, 0u, 0u};
     }
   };
   auto store_stage = [&](int s) {
     unsigned char* st = smem + s * STAGE;
 #pragma unroll
     for (int b = 0; b < ABLK; ++b) *reinterpret_cast<u32x4_t*>(st + b * 4096 + 16 * t) = ld[b];
-    if constexpr (Q4) {
-      // nibbles [block][lane] 16 bytes each, then (scale, bias) words [block][32]
-      *reinterpret_cast<u32x4_t*>(st + ABLK * 4096 + 16 * t) = ld[ABLK];
-      if (t < 32) *reinterpret_cast<u32x4_t*>(st + ABLK * 4096 + 4096 + 16 * t) = ld[ABLK + 1];
-    } else {
-#pragma unroll
-      for (int b = 0; b < 4; ++b) *reinterpret_cast<u32x4_t*>(st + (ABLK + b) * 4096 + 16 * t) = ld[ABLK + b];
-    }
+    // nibbles [block][lane] 16 bytes each, then (scale, bias) words [block][32]
+    *reinterpret_cast<u32x4_t*>(st + ABLK * 4096 + 16 * t) = ld[ABLK];
+    if (t < 32) *reinterpret_cast<u32x4_t*>(st + ABLK * 4096 + 4096 + 16 * t) = ld[ABLK + 1];
   };
   f32x16_t acc[2][2];
 #pragma unroll
@@ -1909,71 +1894,45 @@ __device__ __forceinline__ void long_gemm_body(const GemmParams& p) {
     const int s = kb & 1;
     if (kb + 1 < nkb) load_stage(kb + 1);
     const unsigned char* st = smem + s * STAGE;
-    if constexpr (Q4) {
-      const u32x4_t ones = u32x4_t{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
-      u32x4_t wq[2];
-      float sc[2], cf[2];
+    const u32x4_t ones = u32x4_t{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+    u32x4_t wq[2];
+    float sc[2], cf[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int cb = 2 * wc + j;
+      wq[j] = *reinterpret_cast<const u32x4_t*>(st + ABLK * 4096 + cb * 1024 + 16 * lane);
+      const uint32_t sbw = *reinterpret_cast<const uint32_t*>(st + ABLK * 4096 + 4096 + (cb * 32 + c) * 4);
+      sc[j] = __uint_as_float(sbw << 16);
+      cf[j] = __uint_as_float(sbw & 0xffff0000u) - 128.f * sc[j];
+    }
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      u32x4_t xa[4][NPL];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int pl = 0; pl < NPL; ++pl)
+          xa[i][pl] = *reinterpret_cast<const u32x4_t*>(st + ((2 * wr + rb) * NPL + pl) * 4096 + (64 * i + lane) * 16);
+      f32x16_t xs;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) xs[r] = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int pl = 0; pl < NPL; ++pl) xs = mfma32(xa[i][pl], ones, xs);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int cb = 2 * wc + j;
-        wq[j] = *reinterpret_cast<const u32x4_t*>(st + ABLK * 4096 + cb * 1024 + 16 * lane);
-        const uint32_t sbw = *reinterpret_cast<const uint32_t*>(st + ABLK * 4096 + 4096 + (cb * 32 + c) * 4);
-        sc[j] = __uint_as_float(sbw << 16);
-        cf[j] = __uint_as_float(sbw & 0xffff0000u) - 128.f * sc[j];
-      }
+        f32x16_t au;
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        u32x4_t xa[4][NPL];
+        for (int r = 0; r < 16; ++r) au[r] = 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) {
+          const u32x4_t bq = q4_pairs(wq[j][i]);
 #pragma unroll
-          for (int pl = 0; pl < NPL; ++pl)
-            xa[i][pl] = *reinterpret_cast<const u32x4_t*>(st + ((2 * wr + rb) * NPL + pl) * 4096 + (64 * i + lane) * 16);
-        f32x16_t xs;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) xs[r] = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int pl = 0; pl < NPL; ++pl) xs = mfma32(xa[i][pl], ones, xs);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          f32x16_t au;
-#pragma unroll
-          for (int r = 0; r < 16; ++r) au[r] = 0.f;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const u32x4_t bq = q4_pairs(wq[j][i]);
-#pragma unroll
-            for (int pl = 0; pl < NPL; ++pl) au = mfma32(xa[i][pl], bq, au);
-          }
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[rb][j][r] = fmaf(cf[j], xs[r], fmaf(sc[j], au[r], acc[rb][j][r]));
+          for (int pl = 0; pl < NPL; ++pl) au = mfma32(xa[i][pl], bq, au);
         }
-      }
-    } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int fo = (64 * i + lane) * 16;
-        u32x4_t b[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const u32x4_t*>(st + (ABLK + 2 * wc + j) * 4096 + fo);
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-          const u32x4_t ah = *reinterpret_cast<const u32x4_t*>(st + ((2 * wr + rb) * NPL) * 4096 + fo);
-          if constexpr (H) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[rb][j] = mfma32_f16(ah, b[j], acc[rb][j]);
-          } else {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[rb][j] = mfma32(ah, b[j], acc[rb][j]);
-          }
-          if (LO) {
-            const u32x4_t al = *reinterpret_cast<const u32x4_t*>(st + ((2 * wr + rb) * NPL + 1) * 4096 + fo);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[rb][j] = mfma32(al, b[j], acc[rb][j]);
-          }
-        }
+        for (int r = 0; r < 16; ++r) acc[rb][j][r] = fmaf(cf[j], xs[r], fmaf(sc[j], au[r], acc[rb][j][r]));
       }
     }
     if (kb + 1 < nkb) store_stage(s ^ 1);
@@ -2006,41 +1965,13 @@ __device__ __forceinline__ void long_gemm_body(const GemmParams& p) {
   }
 }
 
-template <bool LO, int EPI, bool H = false>
-__global__ __launch_bounds__(kThreads) void long_gemm_kernel(GemmParams p) {
-  long_gemm_body<LO, EPI, false, H>(p);
-}
-
-template <bool LO, int EPI>
-__global__ __launch_bounds__(kThreads) void longq_gemm_kernel(GemmParams p) {
-  long_gemm_body<LO, EPI, true>(p);
-}
-
 template <bool LO>
-static void launch_long(const GemmParams& p, int epi, int grid, bool q4, bool h16, hipStream_t st) {
-  if (h16) {
-    switch (epi) {
-      case DTREE_EPI_STORE_F32: long_gemm_kernel<false, DTREE_EPI_STORE_F32, true><<<grid, kThreads, 0, st>>>(p); break;
-      case DTREE_EPI_RESIDUAL: long_gemm_kernel<false, DTREE_EPI_RESIDUAL, true><<<grid, kThreads, 0, st>>>(p); break;
-      case DTREE_EPI_SWIGLU: long_gemm_kernel<false, DTREE_EPI_SWIGLU, true><<<grid, kThreads, 0, st>>>(p); break;
-      default: long_gemm_kernel<false, DTREE_EPI_STORE_BF16, true><<<grid, kThreads, 0, st>>>(p); break;
-    }
-    return;
-  }
-  if (q4) {
-    switch (epi) {
-      case DTREE_EPI_STORE_F32: longq_gemm_kernel<LO, DTREE_EPI_STORE_F32><<<grid, kThreads, 0, st>>>(p); break;
-      case DTREE_EPI_RESIDUAL: longq_gemm_kernel<LO, DTREE_EPI_RESIDUAL><<<grid, kThreads, 0, st>>>(p); break;
-      case DTREE_EPI_SWIGLU: longq_gemm_kernel<LO, DTREE_EPI_SWIGLU><<<grid, kThreads, 0, st>>>(p); break;
-      default: longq_gemm_kernel<LO, DTREE_EPI_STORE_BF16><<<grid, kThreads, 0, st>>>(p); break;
-    }
-    return;
-  }
+static void launch_longq(const GemmParams& p, int epi, int grid, hipStream_t st) {
   switch (epi) {
-    case DTREE_EPI_STORE_F32: long_gemm_kernel<LO, DTREE_EPI_STORE_F32><<<grid, kThreads, 0, st>>>(p); break;
-    case DTREE_EPI_RESIDUAL: long_gemm_kernel<LO, DTREE_EPI_RESIDUAL><<<grid, kThreads, 0, st>>>(p); break;
-    case DTREE_EPI_SWIGLU: long_gemm_kernel<LO, DTREE_EPI_SWIGLU><<<grid, kThreads, 0, st>>>(p); break;
-    default: long_gemm_kernel<LO, DTREE_EPI_STORE_BF16><<<grid, kThreads, 0, st>>>(p); break;
+    case DTREE_EPI_STORE_F32: longq_gemm_kernel<LO, DTREE_EPI_STORE_F32><<<grid, kThreads, 0, st>>>(p); break;
+    case DTREE_EPI_RESIDUAL: longq_gemm_kernel<LO, DTREE_EPI_RESIDUAL><<<grid, kThreads, 0, st>>>(p); break;
+    case DTREE_EPI_SWIGLU: longq_gemm_kernel<LO, DTREE_EPI_SWIGLU><<<grid, kThreads, 0, st>>>(p); break;
+    default: longq_gemm_kernel<LO, DTREE_EPI_STORE_BF16><<<grid, kThreads, 0, st>>>(p); break;
   }
 }
 
@@ -2326,6 +2257,22 @@ extern "C" int dtree_gemm_long(const DtreeGemmArgs* a, hipStream_t stream) {
   }
   DTREE_REQUIRE(((uintptr_t)a->x & 15) == 0 && ((uintptr_t)a->x_lo & 15) == 0 && ((uintptr_t)a->w & 15) == 0,
                 "gemm_long: x, x_lo and w must be 16-byte aligned");
+  if (!q4) {
+    LongParams l{};
+    l.x = a->x; l.x_lo = h16 ? nullptr : a->x_lo; l.w = a->w; l.rows = a->rows_padded; l.n = a->n; l.k = a->k;
+    l.ss_in = a->ss_in; l.ss_tiles = a->ss_tiles;
+    l.inv_norm_dim = a->norm_dim > 0 ? 1.0f / (float)a->norm_dim : 1.f; l.eps = a->eps;
+    l.out_f32 = a->out_f32; l.ld_out_f32 = a->ld_out_f32;
+    l.out_tiled = a->out_layout == DTREE_W_TILED || a->out_layout == DTREE_W_TILED_F16;
+    l.out_h16 = a->out_layout == DTREE_W_TILED_F16;
+    l.out_bf16 = a->out_bf16; l.out_lo = l.out_h16 ? nullptr : a->out_lo; l.ld_out_bf16 = a->ld_out_bf16;
+    l.next_norm = a->next_norm; l.ss_out = a->ss_out;
+    l.hidden_out = a->hidden_out; l.ld_hidden = a->ld_hidden;
+    l.vec = ((uintptr_t)a->out_f32 & 15) == 0 && a->ld_out_f32 % 4 == 0 &&
+            ((uintptr_t)a->out_bf16 & 7) == 0 && ((uintptr_t)a->out_lo & 7) == 0 && a->ld_out_bf16 % 4 == 0 &&
+            ((uintptr_t)a->hidden_out & 7) == 0 && a->ld_hidden % 4 == 0 && ((uintptr_t)a->next_norm & 7) == 0;
+    return launch_long_dense(l, epi, h16, device_cus(), stream);
+  }
   GemmParams p{};
   p.x = a->x; p.x_lo = h16 ? nullptr : a->x_lo; p.ldx = a->ldx; p.w = a->w; p.n = a->n; p.k = a->k;
   p.ss_in = a->ss_in; p.ss_tiles = a->ss_tiles;
@@ -2339,8 +2286,8 @@ extern "C" int dtree_gemm_long(const DtreeGemmArgs* a, hipStream_t stream) {
   const long long grid = (long long)(a->rows_padded / kLongRows) * ((a->n + kLongCols - 1) / kLongCols);
   DTREE_REQUIRE(grid < (1LL << 31), "gemm_long: grid too large");
   p.w_sb = a->w_scales;
-  if (p.x_lo) launch_long<true>(p, epi, (int)grid, q4, h16, stream);
-  else launch_long<false>(p, epi, (int)grid, q4, h16, stream);
+  if (p.x_lo) launch_longq<true>(p, epi, (int)grid, stream);
+  else launch_longq<false>(p, epi, (int)grid, stream);
   DTREE_LAUNCH_CHECK("gemm_long launch");
   return DTREE_OK;
 }

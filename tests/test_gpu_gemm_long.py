@@ -1,0 +1,108 @@
+"""dtree_gemm_long's tile shapes against a float64 product.
+
+The fp16 path picks one of six tile shapes by rows and columns; the cases
+below reach every one of them, with ragged last row and column tiles, with
+fewer K stages than the pipeline holds, and with outputs too misaligned for
+the vector stores. Bounds: the fp32 accumulation of K products differs from
+the exact sum by at most K 2^-24 sum |x w| (checked in the result's units);
+fp16 and bf16 outputs add their own rounding (2^-11, 2^-8 relative)."""
+import ctypes as C
+
+import pytest
+import torch
+
+from dtree_hip import _native as N
+from dtree_hip.weights import tile_weight_f16, untile_weight
+
+pytestmark = pytest.mark.gpu
+
+
+def _silu(t):
+    return t * torch.sigmoid(t)
+
+
+def _long(dev, rows, n, k, epi, misaligned=False, seed=0):
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed + rows + 3 * n + 7 * k)
+    x = torch.empty(rows, k, device=dev).normal_(generator=g).half()
+    w = torch.empty(n, k, device=dev).normal_(0.0, 0.05, generator=g).half()
+    xt, wt = tile_weight_f16(x), tile_weight_f16(w)
+    off = 1 if misaligned else 0  # rows of odd length from an odd element: no vector access is aligned
+    width = n // 2 if epi == N.EPI_SWIGLU else n
+    ld = width + off
+    a = N.GemmArgs()
+    a.x = xt.data_ptr(); a.w = wt.data_ptr(); a.x_layout = a.w_layout = N.W_TILED_F16
+    a.ldx = k; a.rows_padded = rows; a.n = n; a.k = k; a.epilogue = epi
+    a.norm_dim = k; a.eps = 1e-6
+    a.out_layout = N.W_ROWMAJOR if misaligned else N.W_TILED_F16
+    f32 = torch.zeros(rows * (n + off) + off, device=dev).normal_(generator=g)
+    res0 = f32[off:].view(rows, n + off)[:, :n].double().clone()
+    act = torch.zeros(rows * ld + off, dtype=torch.int16, device=dev)
+    hid = torch.zeros(rows * (n + off) + off, dtype=torch.bfloat16, device=dev)
+    norm = (1 + 0.1 * torch.empty(n, device=dev).normal_(generator=g)).to(torch.bfloat16)
+    ss = torch.rand(rows // 32, k // 32, 32, device=dev, generator=g) + 0.5
+    sso = torch.zeros(rows // 32, n // 32, 32, device=dev)
+    a.out_f32 = f32.data_ptr() + 4 * off; a.ld_out_f32 = n + off
+    a.out_bf16 = act.data_ptr() + 2 * off; a.ld_out_bf16 = ld
+    rs = torch.ones(rows, dtype=torch.float64, device=dev)
+    if epi == N.EPI_RESIDUAL:
+        a.next_norm = norm.data_ptr(); a.ss_out = sso.data_ptr()
+        a.hidden_out = hid.data_ptr() + 2 * off; a.ld_hidden = n + off
+    else:
+        a.ss_in = ss.data_ptr(); a.ss_tiles = k // 32
+        rs = torch.rsqrt(ss.double().transpose(1, 2).reshape(rows, -1).sum(1) / k + 1e-6)
+    print(f"gemm_long rows={rows} n={n} k={k} epi={epi} misaligned={misaligned}", flush=True)
+    N.check(N.lib().dtree_gemm_long(C.byref(a), torch.cuda.current_stream().cuda_stream), "gemm_long")
+    torch.cuda.synchronize()
+    acc = x.double() @ w.double().T
+    bound = (x.double().abs() @ w.double().abs().T).max().item() * k * 2.0 ** -24 * rs.max().item() + 1e-6
+    f = f32[off:].view(rows, n + off)[:, :n].double()
+    if misaligned:  # row-major bf16
+        b = act[off:].view(rows, ld)[:, :width].view(torch.bfloat16).double()
+        rnd = 2.0 ** -8
+    else:
+        b = untile_weight(act.view(torch.float16).view(rows, width)).double()
+        rnd = 2.0 ** -11
+    if epi == N.EPI_STORE_F32:
+        assert (f - acc * rs[:, None]).abs().max().item() <= bound
+    elif epi == N.EPI_STORE_BF16:
+        ref = acc * rs[:, None]
+        assert ((b - ref).abs() <= bound + rnd * ref.abs() + 2.0 ** -24).all()
+    elif epi == N.EPI_SWIGLU:
+        v = (acc * rs[:, None]).reshape(rows, n // 32, 2, 16)
+        ga, up = v[:, :, 0].reshape(rows, -1), v[:, :, 1].reshape(rows, -1)
+        ref = _silu(ga) * up
+        # |silu'| <= 1.1; the device's exp and divide are within a few ulp
+        err = bound * (1.1 * up.abs() + ga.abs()) + 1e-6 * ref.abs()
+        assert ((b - ref).abs() <= err + rnd * ref.abs() + 2.0 ** -24).all()
+    else:
+        ref = res0 + acc
+        assert (f - ref).abs().max().item() <= bound + 2.0 ** -23 * ref.abs().max().item()
+        xg = f * norm.double()
+        assert ((b - xg).abs() <= (rnd + 1e-6) * xg.abs() + 2.0 ** -24).all()
+        h = hid[off:].view(rows, n + off)[:, :n]
+        assert torch.equal(h, f.float().to(torch.bfloat16))
+        want = f.square().reshape(rows // 32, 32, n // 32, 32).sum(-1).transpose(1, 2)
+        torch.testing.assert_close(sso.double(), want, rtol=1e-5, atol=1e-5)
+
+
+# (rows, n): 128x128 (K halves), 256x128, 256x192, 256x256, 256x320, 256x384 tiles
+SHAPES = [(128, 256), (1152, 6144), (640, 19456), (1152, 12416), (1024, 19456), (1152, 24576)]
+
+
+@pytest.mark.parametrize("rows,n", SHAPES)
+@pytest.mark.parametrize("epi", [N.EPI_STORE_F32, N.EPI_RESIDUAL, N.EPI_SWIGLU, N.EPI_STORE_BF16])
+@pytest.mark.parametrize("k", [64, 320])
+def test_long_tiles_match_float64(gpu_device, rows, n, epi, k):
+    _long(gpu_device, rows, n, k, epi)
+
+
+@pytest.mark.parametrize("rows,n", [(128, 64), (1024, 12352), (640, 19520), (1024, 19520), (1152, 24640)])
+def test_long_tiles_64_column_tail(gpu_device, rows, n):
+    _long(gpu_device, rows, n, 192, N.EPI_STORE_F32)
+
+
+@pytest.mark.parametrize("rows,n", [(384, 256), (1152, 6144), (1024, 19456)])
+@pytest.mark.parametrize("epi", [N.EPI_STORE_F32, N.EPI_RESIDUAL, N.EPI_SWIGLU, N.EPI_STORE_BF16])
+def test_long_tiles_misaligned_outputs(gpu_device, rows, n, epi):
+    _long(gpu_device, rows, n, 128, epi, misaligned=True)
