@@ -1812,169 +1812,6 @@ static void launch_dp_any(const GemmParams& p, int epi, bool q4, bool h16, hipSt
   else lo ? launch_dp<true, KS, false>(p, epi, st) : launch_dp<false, KS, false>(p, epi, st);
 }
 
-// ---- long-M GEMM (prompt prefill), q4 weights: rows a multiple of 128 --------
-// Compute-bound: a workgroup owns a 128-row x 128-column output tile over the
-// whole K. A K block (64) is one quantisation group; per block the workgroup
-// stages the tile's activation blocks (4 row blocks, hi and lo planes), 1 KB
-// of nibbles and 32 (scale, bias) words per 32-column block in LDS,
-// double-buffered with one barrier per K block (the next block's loads are in
-// flight during the current block's MFMAs). Wave w computes rows 64 (w / 2) ..
-// + 63 x columns 64 (w % 2) .. + 63 as 2 x 2 MFMA 32 x 32 tiles: each takes a
-// fresh MFMA sum of x (128 + q) per group and folds it in as acc += s * sum +
-// (b - 128 s) * sum(x), with sum(x) per row block from an MFMA of the staged
-// activations against bf16 ones. The finished tile goes through LDS to the
-// same epilogues as the skinny GEMMs, applied to 128 rows.
-constexpr int kLongRows = 128, kLongCols = 128;
-
-template <bool LO, int EPI>
-__global__ __launch_bounds__(kThreads) void longq_gemm_kernel(GemmParams p) {
-  constexpr int NPL = LO ? 2 : 1, ABLK = 4 * NPL;
-  constexpr int WBYTES = 4 * 1024 + 4 * 128;                            // weight bytes per stage
-  constexpr int STAGE = ABLK * 4096 + WBYTES;                           // bytes per stage
-  constexpr int SMEM = 2 * STAGE > kLongRows * kLongCols * 4 ? 2 * STAGE : kLongRows * kLongCols * 4;
-  __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM];
-  __shared__ float rs[kLongRows];
-  const int t = threadIdx.x, lane = t & 63, c = lane & 31, h = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int wr = wave >> 1, wc = wave & 1;
-  const int ntn = (p.n + kLongCols - 1) / kLongCols;  // the last tile may hold 64 columns (STORE_F32)
-  const int mt = blockIdx.x / ntn, nt = blockIdx.x - mt * ntn;
-  const int nkb = p.k >> 6;
-  const int R = mt * kLongRows;
-  if (t < kLongRows) {
-    float r = 1.f;
-    if (p.ss_in) {
-      float s = 0.f;
-      for (int tt = 0; tt < p.ss_tiles; ++tt) s += p.ss_in[ss_index(tt, R + t, p.ss_tiles)];
-      r = rsqrtf(s * p.inv_norm_dim + p.eps);
-    }
-    rs[t] = r;
-  }
-  // Staged per thread: ABLK activation pieces, then 16 bytes of nibbles, and
-  // for t < 32 16 bytes of scale / bias words.
-  constexpr int NW = 2;
-  u32x4_t ld[ABLK + NW];
-  const uint32_t* wsb = reinterpret_cast<const uint32_t*>(p.w_sb);
-  auto load_stage = [&](int kb) {
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-      const size_t blk = ((size_t)((R >> 5) + rb) * nkb + kb) * 2048 + 8 * t;
-      ld[rb * NPL] = ld_u32x4(p.x + blk);
-      if (LO) ld[rb * NPL + NPL - 1] = ld_u32x4(p.x_lo + blk);
-    }
-    const int cb = nt * 4 + (t >> 6);  // this thread's 32-column block
-    ld[ABLK] = cb * 32 < p.n ? ld_u32x4(reinterpret_cast<const uint32_t*>(p.w) + ((size_t)cb * nkb + kb) * 256 +
-                                        4 * (t & 63))
-                             : u32x4_t{0u, 0u, 0u, 0u};
-    if (t < 32) {
-      const int sbb = nt * 4 + (t >> 3);
-      ld[ABLK + 1] = sbb * 32 < p.n ? ld_u32x4(wsb + ((size_t)sbb * nkb + kb) * 32 + 4 * (t & 7))
-                                    : u32x4_t{0u, 0u, 0u, 0u};
-    }
-  };
-  auto store_stage = [&](int s) {
-    unsigned char* st = smem + s * STAGE;
-#pragma unroll
-    for (int b = 0; b < ABLK; ++b) *reinterpret_cast<u32x4_t*>(st + b * 4096 + 16 * t) = ld[b];
-    // nibbles [block][lane] 16 bytes each, then (scale, bias) words [block][32]
-    *reinterpret_cast<u32x4_t*>(st + ABLK * 4096 + 16 * t) = ld[ABLK];
-    if (t < 32) *reinterpret_cast<u32x4_t*>(st + ABLK * 4096 + 4096 + 16 * t) = ld[ABLK + 1];
-  };
-  f32x16_t acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  load_stage(0);
-  store_stage(0);
-  __syncthreads();
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int s = kb & 1;
-    if (kb + 1 < nkb) load_stage(kb + 1);
-    const unsigned char* st = smem + s * STAGE;
-    const u32x4_t ones = u32x4_t{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
-    u32x4_t wq[2];
-    float sc[2], cf[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int cb = 2 * wc + j;
-      wq[j] = *reinterpret_cast<const u32x4_t*>(st + ABLK * 4096 + cb * 1024 + 16 * lane);
-      const uint32_t sbw = *reinterpret_cast<const uint32_t*>(st + ABLK * 4096 + 4096 + (cb * 32 + c) * 4);
-      sc[j] = __uint_as_float(sbw << 16);
-      cf[j] = __uint_as_float(sbw & 0xffff0000u) - 128.f * sc[j];
-    }
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      u32x4_t xa[4][NPL];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int pl = 0; pl < NPL; ++pl)
-          xa[i][pl] = *reinterpret_cast<const u32x4_t*>(st + ((2 * wr + rb) * NPL + pl) * 4096 + (64 * i + lane) * 16);
-      f32x16_t xs;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) xs[r] = 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int pl = 0; pl < NPL; ++pl) xs = mfma32(xa[i][pl], ones, xs);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        f32x16_t au;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) au[r] = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const u32x4_t bq = q4_pairs(wq[j][i]);
-#pragma unroll
-          for (int pl = 0; pl < NPL; ++pl) au = mfma32(xa[i][pl], bq, au);
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[rb][j][r] = fmaf(cf[j], xs[r], fmaf(sc[j], au[r], acc[rb][j][r]));
-      }
-    }
-    if (kb + 1 < nkb) store_stage(s ^ 1);
-    __syncthreads();
-  }
-  float* red = reinterpret_cast<float*>(smem);
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        red[(64 * wr + 32 * rb + acc_row(r, h)) * kLongCols + 64 * wc + 32 * j + c] = acc[rb][j][r];
-  __syncthreads();
-  // The epilogue of rows R .. R + 127, one 32-row block at a time (outputs
-  // shifted by the block's first row: 32-row blocks are contiguous in both
-  // layouts; statistics are per 32-row block). In one 128-row piece the
-  // residual epilogue held 64 preloaded values per thread and took the kernel
-  // to 320 VGPRs, one workgroup per CU for the whole K loop.
-#pragma unroll 1
-  for (int r2 = 0; r2 < kLongRows / 32; ++r2) {
-    const int R2 = R + 32 * r2;
-    GemmParams q = p;
-    if (q.out_f32) q.out_f32 += (size_t)R2 * q.ld_out_f32;
-    if (q.out_bf16) q.out_bf16 += (size_t)R2 * q.ld_out_bf16;
-    if (q.out_lo) q.out_lo += (size_t)R2 * q.ld_out_bf16;
-    if (q.hidden_out) q.hidden_out += (size_t)R2 * q.ld_hidden;
-    if (q.ss_out) q.ss_out += (size_t)(R2 >> 5) * (q.n >> 5) * 32;
-    tile_epilogue<32, kLongCols, EPI>(q, red + 32 * r2 * kLongCols, rs + 32 * r2, nt);
-  }
-}
-
-template <bool LO>
-static void launch_longq(const GemmParams& p, int epi, int grid, hipStream_t st) {
-  switch (epi) {
-    case DTREE_EPI_STORE_F32: longq_gemm_kernel<LO, DTREE_EPI_STORE_F32><<<grid, kThreads, 0, st>>>(p); break;
-    case DTREE_EPI_RESIDUAL: longq_gemm_kernel<LO, DTREE_EPI_RESIDUAL><<<grid, kThreads, 0, st>>>(p); break;
-    case DTREE_EPI_SWIGLU: longq_gemm_kernel<LO, DTREE_EPI_SWIGLU><<<grid, kThreads, 0, st>>>(p); break;
-    default: longq_gemm_kernel<LO, DTREE_EPI_STORE_BF16><<<grid, kThreads, 0, st>>>(p); break;
-  }
-}
-
 }  // namespace dtree
 
 using namespace dtree;
@@ -2220,6 +2057,8 @@ extern "C" int dtree_gemm_bf16(const DtreeGemmArgs* a, hipStream_t stream) {
   return DTREE_OK;
 }
 
+constexpr int kLongAlign = 128;  // rows of a long GEMM come in multiples of this
+
 extern "C" int dtree_gemm_long(const DtreeGemmArgs* a, hipStream_t stream) {
   DTREE_REQUIRE(a, "gemm_long: null args");
   DTREE_REQUIRE(a->x && a->w, "gemm_long: null x or w");
@@ -2230,10 +2069,10 @@ extern "C" int dtree_gemm_long(const DtreeGemmArgs* a, hipStream_t stream) {
                 "gemm_long: tiled bf16 activations with tiled bf16 or q4 group-64 weights, or TILED_F16 both");
   DTREE_REQUIRE(!q4 || (a->w_scales && ((uintptr_t)a->w_scales & 15) == 0),
                 "gemm_long: q4 weights need w_scales (16-byte aligned)");
-  DTREE_REQUIRE(a->rows_padded >= kLongRows && a->rows_padded % kLongRows == 0 && a->rows_padded <= (1 << 20),
+  DTREE_REQUIRE(a->rows_padded >= kLongAlign && a->rows_padded % kLongAlign == 0 && a->rows_padded <= (1 << 20),
                 "gemm_long: rows_padded must be a positive multiple of 128");
   const int epi = a->epilogue;
-  DTREE_REQUIRE(a->n > 0 && (a->n % kLongCols == 0 || (a->n % 64 == 0 && epi == DTREE_EPI_STORE_F32)),
+  DTREE_REQUIRE(a->n > 0 && (a->n % 128 == 0 || (a->n % 64 == 0 && epi == DTREE_EPI_STORE_F32)),
                 "gemm_long: n must be a positive multiple of 128 (of 64 with the fp32 store epilogue)");
   DTREE_REQUIRE(a->k > 0 && a->k % 64 == 0 && a->ldx == a->k, "gemm_long: k a multiple of 64, ldx == k");
   DTREE_REQUIRE(epi >= 0 && epi <= 3, "gemm_long: unknown epilogue");
@@ -2257,39 +2096,20 @@ extern "C" int dtree_gemm_long(const DtreeGemmArgs* a, hipStream_t stream) {
   }
   DTREE_REQUIRE(((uintptr_t)a->x & 15) == 0 && ((uintptr_t)a->x_lo & 15) == 0 && ((uintptr_t)a->w & 15) == 0,
                 "gemm_long: x, x_lo and w must be 16-byte aligned");
-  if (!q4) {
-    LongParams l{};
-    l.x = a->x; l.x_lo = h16 ? nullptr : a->x_lo; l.w = a->w; l.rows = a->rows_padded; l.n = a->n; l.k = a->k;
-    l.ss_in = a->ss_in; l.ss_tiles = a->ss_tiles;
-    l.inv_norm_dim = a->norm_dim > 0 ? 1.0f / (float)a->norm_dim : 1.f; l.eps = a->eps;
-    l.out_f32 = a->out_f32; l.ld_out_f32 = a->ld_out_f32;
-    l.out_tiled = a->out_layout == DTREE_W_TILED || a->out_layout == DTREE_W_TILED_F16;
-    l.out_h16 = a->out_layout == DTREE_W_TILED_F16;
-    l.out_bf16 = a->out_bf16; l.out_lo = l.out_h16 ? nullptr : a->out_lo; l.ld_out_bf16 = a->ld_out_bf16;
-    l.next_norm = a->next_norm; l.ss_out = a->ss_out;
-    l.hidden_out = a->hidden_out; l.ld_hidden = a->ld_hidden;
-    l.vec = ((uintptr_t)a->out_f32 & 15) == 0 && a->ld_out_f32 % 4 == 0 &&
-            ((uintptr_t)a->out_bf16 & 7) == 0 && ((uintptr_t)a->out_lo & 7) == 0 && a->ld_out_bf16 % 4 == 0 &&
-            ((uintptr_t)a->hidden_out & 7) == 0 && a->ld_hidden % 4 == 0 && ((uintptr_t)a->next_norm & 7) == 0;
-    return launch_long_dense(l, epi, h16, device_cus(), stream);
-  }
-  GemmParams p{};
-  p.x = a->x; p.x_lo = h16 ? nullptr : a->x_lo; p.ldx = a->ldx; p.w = a->w; p.n = a->n; p.k = a->k;
-  p.ss_in = a->ss_in; p.ss_tiles = a->ss_tiles;
-  p.inv_norm_dim = a->norm_dim > 0 ? 1.0f / (float)a->norm_dim : 1.f; p.eps = a->eps;
-  p.out_f32 = a->out_f32; p.ld_out_f32 = a->ld_out_f32;
-  p.out_tiled = a->out_layout == DTREE_W_TILED || a->out_layout == DTREE_W_TILED_F16;
-  p.out_h16 = a->out_layout == DTREE_W_TILED_F16;
-  p.out_bf16 = a->out_bf16; p.out_lo = p.out_h16 ? nullptr : a->out_lo; p.ld_out_bf16 = a->ld_out_bf16;
-  p.next_norm = a->next_norm; p.ss_out = a->ss_out;
-  p.hidden_out = a->hidden_out; p.ld_hidden = a->ld_hidden;
-  const long long grid = (long long)(a->rows_padded / kLongRows) * ((a->n + kLongCols - 1) / kLongCols);
-  DTREE_REQUIRE(grid < (1LL << 31), "gemm_long: grid too large");
-  p.w_sb = a->w_scales;
-  if (p.x_lo) launch_longq<true>(p, epi, (int)grid, stream);
-  else launch_longq<false>(p, epi, (int)grid, stream);
-  DTREE_LAUNCH_CHECK("gemm_long launch");
-  return DTREE_OK;
+  LongParams l{};
+  l.x = a->x; l.x_lo = h16 ? nullptr : a->x_lo; l.w = a->w; l.w_sb = a->w_scales; l.rows = a->rows_padded; l.n = a->n; l.k = a->k;
+  l.ss_in = a->ss_in; l.ss_tiles = a->ss_tiles;
+  l.inv_norm_dim = a->norm_dim > 0 ? 1.0f / (float)a->norm_dim : 1.f; l.eps = a->eps;
+  l.out_f32 = a->out_f32; l.ld_out_f32 = a->ld_out_f32;
+  l.out_tiled = a->out_layout == DTREE_W_TILED || a->out_layout == DTREE_W_TILED_F16;
+  l.out_h16 = a->out_layout == DTREE_W_TILED_F16;
+  l.out_bf16 = a->out_bf16; l.out_lo = l.out_h16 ? nullptr : a->out_lo; l.ld_out_bf16 = a->ld_out_bf16;
+  l.next_norm = a->next_norm; l.ss_out = a->ss_out;
+  l.hidden_out = a->hidden_out; l.ld_hidden = a->ld_hidden;
+  l.vec = ((uintptr_t)a->out_f32 & 15) == 0 && a->ld_out_f32 % 4 == 0 &&
+          ((uintptr_t)a->out_bf16 & 7) == 0 && ((uintptr_t)a->out_lo & 7) == 0 && a->ld_out_bf16 % 4 == 0 &&
+          ((uintptr_t)a->hidden_out & 7) == 0 && a->ld_hidden % 4 == 0 && ((uintptr_t)a->next_norm & 7) == 0;
+  return q4 ? launch_long_q4(l, epi, device_cus(), stream) : launch_long_dense(l, epi, h16, device_cus(), stream);
 }
 
 extern "C" size_t dtree_lmhead_candidates_bytes(int32_t rows_padded) {

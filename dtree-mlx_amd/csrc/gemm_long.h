@@ -6,7 +6,7 @@ namespace dtree {
 
 struct LongParams {
   const uint16_t* x; const uint16_t* x_lo;
-  const uint16_t* w; int rows, n, k;
+  const uint16_t* w; const uint16_t* w_sb; int rows, n, k;  // w_sb: q4 (scale, bias) pairs
   const float* ss_in; int ss_tiles; float inv_norm_dim; float eps;
   float* out_f32; int ld_out_f32;
   uint16_t* out_bf16; uint16_t* out_lo; int ld_out_bf16; int out_tiled;
@@ -21,5 +21,6 @@ struct LongParams {
 // Dense weights (bf16 with an optional low activation plane, or fp16); ntn and
 // tiles are filled in here.
 int launch_long_dense(LongParams p, int epi, bool h16, int cus, hipStream_t st);
+int launch_long_q4(LongParams p, int epi, int cus, hipStream_t st);
 
 }  // namespace dtree

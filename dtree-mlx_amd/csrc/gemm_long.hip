@@ -1,5 +1,5 @@
 // Long-M GEMM Y[M, N] = X[M, K] * W[N, K]^T for the prompt prefill (rows a
-// multiple of 128), dense weights. Compute-bound: the design goal is MFMA
+// multiple of 128). Compute-bound: the design goal is MFMA
 // issue, so the tile, not the weight stream, is what each workgroup shares.
 //
 // * Both operands are in the tiled layout (32-row x 64-column blocks, four
@@ -64,7 +64,7 @@ __device__ __forceinline__ void lds_load16(u32x4_t r, unsigned off, unsigned lds
 // then the workgroup barrier.
 template <int N>
 __device__ __forceinline__ void stage_wait() {
-  static_assert(N <= 63, "vmcnt is 6 bits");
+  static_assert(N >= 0 && N <= 63, "vmcnt is 6 bits");
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
 }
 
@@ -197,6 +197,62 @@ __device__ __forceinline__ void long_epilogue(const LongParams& p, f32x16_t (&ac
         }
       }
     }
+  }
+}
+
+// Epilogues of the workgroup's finished accumulators (the stages' LDS is free
+// again after the first barrier in here). With KS = 2 the waves of a pair swap
+// half of their row blocks through LDS, and each adds and finishes the half it
+// keeps. `turn` brings acc[j][i] into the epilogue's layout in place if the
+// kernel accumulates another one; its scratch is 32 x 36 floats per wave.
+template <class T, int EPI, class Turn>
+__device__ __forceinline__ void long_finish(const LongParams& p, f32x16_t (&acc)[T::NB][T::MB], unsigned char* smem,
+                                            const float* rs, int wave, int R, int N0, Turn turn) {
+  constexpr int MB = T::MB, NB = T::NB;
+  const int lane = threadIdx.x & 63;
+  const int kg = T::KS > 1 ? wave / (T::GM * T::GN) : 0, wt = wave - kg * (T::GM * T::GN);
+  const int wm = wt / T::GN, wn = wt % T::GN;
+  const int mw = 32 * MB * wm, n0 = N0 + 32 * NB * wn;
+  float* scratch = reinterpret_cast<float*>(smem) + wave * (32 * 36);
+  stage_wait<0>();  // every wave's loads and reads of the stages are done
+  if constexpr (T::KS > 1) {
+    static_assert(MB % 2 == 0, "a pair of waves swaps half of its row blocks");
+    constexpr int HB = MB / 2;
+    f32x4_t* ex = reinterpret_cast<f32x4_t*>(smem) + (size_t)wt * (2 * NB * HB * 256) + lane;
+    auto slot = [&](int g, int j, int i, int q) { return ex + (((g * NB + j) * HB + i) * 4 + q) * 64; };
+    f32x16_t half[NB][HB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < HB; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          f32x4_t v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = kg ? acc[j][i][4 * q + e] : acc[j][HB + i][4 * q + e];
+          *slot(kg, j, i, q) = v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) half[j][i][4 * q + e] = kg ? acc[j][HB + i][4 * q + e] : acc[j][i][4 * q + e];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int i = 0; i < HB; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4_t v = *slot(1 - kg, j, i, q);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) half[j][i][4 * q + e] += v[e];
+        }
+    __syncthreads();
+    turn(half, scratch);
+    if (p.vec) long_epilogue<NB, HB, EPI, true>(p, half, rs, R, mw + 32 * HB * kg, n0);
+    else long_epilogue<NB, HB, EPI, false>(p, half, rs, R, mw + 32 * HB * kg, n0);
+  } else {
+    turn(acc, scratch);
+    if (p.vec) long_epilogue<NB, MB, EPI, true>(p, acc, rs, R, mw, n0);
+    else long_epilogue<NB, MB, EPI, false>(p, acc, rs, R, mw, n0);
   }
 }
 
@@ -338,67 +394,354 @@ __global__ __launch_bounds__(T::THREADS) void long_kernel(LongParams p) {
       step(s, f);
     }
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into this LDS outlives the workgroup
-  const int mw = 32 * MB * wm, n0 = N0 + 32 * NB * wn;
-  if constexpr (KS > 1) {
-    // The two K halves: the waves of a pair swap half of their row blocks
-    // through LDS, each adds and finishes the half it keeps.
-    static_assert(MB % 2 == 0 && T::GM * T::GN * NB * MB * 4096 <= NST * STAGE, "the exchange fits the stages");
-    constexpr int HB = MB / 2;
-    stage_wait<0>();  // every wave's loads and reads of the stages are done
-    f32x4_t* ex = reinterpret_cast<f32x4_t*>(smem) + (size_t)wt * (2 * NB * HB * 256) + lane;
-    auto slot = [&](int g, int j, int i, int q) { return ex + (((g * NB + j) * HB + i) * 4 + q) * 64; };
-    f32x16_t half[NB][HB];
+  long_finish<T, EPI>(p, acc, smem, rs, wave, R, N0, [](auto&, float*) {});
+}
+
+// ---- q4 group-64 weights ---------------------------------------------------------
+// The same tiles and pipeline over 4-bit weights with bf16 activations. A K
+// block is one quantisation group and one stage (per K group of the tile): the
+// activation fragments, 1 KB of nibbles and 32 (scale, bias) words per column
+// block, all by direct loads.
+//
+// y = sum_g s_g sum_k x_k q_k + b_g sum_k x_k. The nibbles enter the MFMA as
+// bf16 128 + q (exact), so per group
+//   acc += s * (x . (128 + q)),  and  acc += (b - 128 s) * sum(x).
+// The first is a fresh four-MFMA sum per 32 x 32 block folded in by one FMA per
+// element, under the next block's MFMAs. The second is a product over the
+// groups, [rows x groups] x [groups x columns], so it runs on MFMA as well, once
+// per eight groups: each group's sum(x) (dot products with ones, one wave per
+// row block) and b - 128 s (one wave per column block) go to an LDS ring as
+// fp32; both are split into three bf16 parts (24 significant bits), and three
+// MFMAs cover the six products down to 2^-16, two of them side by side in the
+// 16 K slots (the lane halves). As FMAs it would cost as many again as the
+// first fold, which with the nibble unpacking is what bounds the kernel.
+//
+// The accumulators are X W^T here (a scale is then one value per lane) and are
+// turned into the epilogues' layout through LDS once per tile.
+//
+// Measured against the kernel this one replaced (128 x 128 tiles through
+// registers, both folds as FMAs, sum(x) by MFMA in every wave): the 9B-shaped
+// MLP (gate/up and down) over 300 tokens 476 -> 248 us; N 24576, K 4096, 4096
+// rows 913 us (0.90 PFLOP/s; the fp16 tiles reach 1.18).
+constexpr int kRing = 8;        // groups per correction step
+constexpr int kRingStride = 12; // floats per ring row (16-byte reads, spread over the banks)
+
+__device__ __forceinline__ u32x4_t q4_pairs16(uint32_t w, uint32_t m, uint32_t e) {
+  return u32x4_t{(w & m) | e, ((w >> 4) & m) | e, ((w >> 8) & m) | e, ((w >> 12) & m) | e};
+}
+
+// Sum of the eight bf16 of w, added to s.
+__device__ __forceinline__ float bf8_sum(u32x4_t w, float s) {
+  const bf16x2_t one = __builtin_bit_cast(bf16x2_t, 0x3f803f80u);
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
+  for (int i = 0; i < 4; ++i)
+    s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, (uint32_t)w[i]), one, s, false);
+  return s;
+}
+
+// a + the other half-wave's a. As row_pair_sum (common.h): one asm sequence,
+// since the compiler folds the two results of the swap of equal registers.
+__device__ __forceinline__ float half_pair_sum(float a) {
+  float b;
+  asm volatile("v_mov_b32 %1, %0\n\ts_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\tv_add_f32 %0, %0, %1"
+               : "+v"(a), "=&v"(b));
+  return a;
+}
+
+// v = hi + mid + lo, each bf16, to about 24 significant bits.
+__device__ __forceinline__ void split3(const float (&v)[8], u32x4_t& hi, u32x4_t& mid, u32x4_t& lo) {
 #pragma unroll
-      for (int i = 0; i < HB; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          f32x4_t v;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = kg ? acc[j][i][4 * q + e] : acc[j][HB + i][4 * q + e];
-          *slot(kg, j, i, q) = v;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) half[j][i][4 * q + e] = kg ? acc[j][HB + i][4 * q + e] : acc[j][i][4 * q + e];
-        }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-#pragma unroll
-      for (int i = 0; i < HB; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x4_t v = *slot(1 - kg, j, i, q);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) half[j][i][4 * q + e] += v[e];
-        }
-    if (p.vec) long_epilogue<NB, HB, EPI, true>(p, half, rs, R, mw + 32 * HB * kg, n0);
-    else long_epilogue<NB, HB, EPI, false>(p, half, rs, R, mw + 32 * HB * kg, n0);
-  } else {
-    if (p.vec) long_epilogue<NB, MB, EPI, true>(p, acc, rs, R, mw, n0);
-    else long_epilogue<NB, MB, EPI, false>(p, acc, rs, R, mw, n0);
+  for (int i = 0; i < 4; ++i) {
+    const float a = v[2 * i], b = v[2 * i + 1];
+    hi[i] = pack_bf2(a, b);
+    const float a1 = a - __uint_as_float(hi[i] << 16), b1 = b - __uint_as_float(hi[i] & 0xffff0000u);
+    mid[i] = pack_bf2(a1, b1);
+    lo[i] = pack_bf2(a1 - __uint_as_float(mid[i] << 16), b1 - __uint_as_float(mid[i] & 0xffff0000u));
   }
 }
 
-template <class T, bool H, int NPL>
+template <class T, int EPI, int NPL>
+__global__ __launch_bounds__(T::THREADS) void longq_kernel(LongParams p) {
+  constexpr int MB = T::MB, NB = T::NB, NST = T::NST, KS = T::KS, WT = T::GM * T::GN;
+  constexpr int RB = T::TM / 32, CB = T::TN / 32;
+  constexpr int PA = RB * NPL * 4, CHK = PA + CB + 1;  // 1 KB pieces per K block: x, nibbles, scale words
+  constexpr int CH = KS * CHK, STAGE = CH * 1024;
+  constexpr int PW = (CH + T::WAVES - 1) / T::WAVES;
+  constexpr bool PAD = CH % T::WAVES != 0;
+  static_assert(CB <= 8, "one piece holds the tile's scale words");
+  static_assert(NST * STAGE >= T::WAVES * 32 * 36 * 4 && (KS == 1 || NST * STAGE >= WT * NB * MB * 4096),
+                "long_finish's scratch");
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[NST * STAGE + (PAD ? 1024 : 0)];
+  __shared__ __attribute__((aligned(16))) float xring[KS][T::TM][kRingStride], cring[KS][T::TN][kRingStride];
+  __shared__ float rs[T::TM];
+  const int t = threadIdx.x, lane = t & 63, c = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int kg = KS > 1 ? wave / WT : 0, wt = wave - kg * WT;
+  const int wm = wt / T::GN, wn = wt % T::GN;
+  const int2 mn = xcd_tile(blockIdx.x, p.tiles, p.ntn, T::TM);
+  const int R = mn.x * T::TM, N0 = mn.y * T::TN;
+  const unsigned nkb = (unsigned)p.k >> 6;
+  const int S = (int)nkb / KS;  // KS = 2 takes an even number of K blocks
+  const unsigned mrb = (unsigned)min(T::TM, p.rows - R) / 32u, ncb = (unsigned)min(T::TN, p.n - N0) / 32u;
+  const size_t xo = (size_t)R * p.k, cb0 = (size_t)(N0 >> 5) * nkb;
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+  // Piece wave + WAVES j of every stage: its strips' base and size, its offset
+  // in stage 0, the offset's step per stage and its place in a stage.
+  // (A piece past the last has size 0, reads nothing and keeps the counts equal.)
+  uint32_t plo[PW], phi[PW], psize[PW], poff[PW], pstep[PW], plds[PW], pstage[PW];
+  uint32_t pmask[PW];
+#pragma unroll
+  for (int j = 0; j < PW; ++j) {
+    const int ch = wave + T::WAVES * j;
+    const int g = KS > 1 ? ch / CHK : 0, q = ch - g * CHK;
+    const bool pad = PAD && ch >= CH;
+    const bool isx = q < PA, isw = !isx && q < PA + CB, low = NPL > 1 && isx && q >= PA / NPL;
+    const int a = isx ? (low ? q - PA / NPL : q) : q - PA;
+    const unsigned kstep = isx ? 4096u : isw ? 1024u : 128u;  // bytes of one K block of a strip
+    const uint64_t base = isx ? (uint64_t)((low ? p.x_lo : p.x) + xo)
+                              : isw ? (uint64_t)(p.w + cb0 * 512) : (uint64_t)(p.w_sb + cb0 * 64);
+    plo[j] = uni((uint32_t)base);
+    phi[j] = uni((uint32_t)(base >> 32) & 0xffffu);
+    psize[j] = uni(pad ? 0u : (isx ? mrb : ncb) * nkb * kstep);
+    poff[j] = uni((isx ? (unsigned)(a >> 2) : isw ? (unsigned)a : 0u) * nkb * kstep + g * kstep +
+                  (isx ? (a & 3) * 1024u : 0u));
+    pstep[j] = uni(KS * kstep);
+    plds[j] = uni(lds0 + (pad ? NST * STAGE : 1024 * ch));
+    pstage[j] = uni(pad ? 0u : ~0u);  // padding has one place for all stages
+    pmask[j] = uni(isx || isw ? 0u : ~0u);  // scale words: eight lanes per column block
+  }
+  const unsigned lane16 = 16u * lane, lane_s = (unsigned)(lane >> 3) * nkb * 128u + 16u * (lane & 7) - lane16;
+  // `at`: the stage's LDS offset. Past the last stage the size is 0 (no branch
+  // and no select: the stage loop stays one block, as its order is written).
+  auto issue = [&](int s, unsigned at, int j) {
+    const uint32_t live = (uint32_t)((s - S) >> 31);
+    lds_load16(u32x4_t{plo[j], phi[j], psize[j] & live, 0x00020000u},
+               poff[j] + (unsigned)s * pstep[j] + lane16 + (lane_s & pmask[j]), plds[j] + (at & pstage[j]));
+  };
+  f32x16_t acc[NB][MB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.f;
+  uint32_t nib_m, nib_e;  // in registers: the three-operand form takes no literal
+  asm("s_mov_b32 %0, 0x000f000f" : "=s"(nib_m));
+  asm("v_mov_b32 %0, 0x43004300" : "=v"(nib_e));
+  constexpr int NT = MB * NB;
+  // row blocks whose sums, and column blocks whose ring entries, a wave makes
+  constexpr int NSUM = MB > T::GN ? MB / T::GN : 1, NCR = (CB + WT - 1) / WT;
+  static_assert((MB % T::GN == 0 || T::GN % MB == 0) && NT % 2 == 0 && 2 * NSUM <= NT - NB && CB % (NCR * 2) == 0,
+                "sums shared out evenly and done before the last row block; running sums alternate");
+  u32x4_t fa[4 * NPL], wq[NB], bq[NB][4];
+  uint32_t sbw[NB], cw[NCR];
+  float sc[NB];
+  f32x16_t au[2];
+  const unsigned char* kbase = smem + kg * (CHK * 1024);
+  auto read_a = [&](unsigned at, int i, int f, int pl) {
+    fa[f * NPL + pl] = *reinterpret_cast<const u32x4_t*>(
+        kbase + at + ((pl * RB + wm * MB + i) * 4 + f) * 1024 + 16 * lane);
+  };
+  auto read_w = [&](unsigned at, int j) {
+    const unsigned char* st = kbase + at + PA * 1024;
+    wq[j] = *reinterpret_cast<const u32x4_t*>(st + (wn * NB + j) * 1024 + 16 * lane);
+    sbw[j] = *reinterpret_cast<const uint32_t*>(st + CB * 1024 + (wn * NB + j) * 128 + 4 * c);
+    if (j < NCR) cw[j] = *reinterpret_cast<const uint32_t*>(st + CB * 1024 + min(wt * NCR + j, CB - 1) * 128 + 4 * c);
+  };
+  auto unpack = [&](int j, int f) {
+    bq[j][f] = q4_pairs16(wq[j][f], nib_m, nib_e);
+  };
+  // sum(x) of the group for this wave's row blocks (both lane halves hold and
+  // write the same value, as do waves that share a row block)
+  const int srow = wm * MB + (MB > T::GN ? wn * NSUM : wn % MB);
+  u32x4_t sx[4 * NPL];
+  float ssum[2];
+  auto sum_read = [&](unsigned at, int e, int f) {
+#pragma unroll
+    for (int pl = 0; pl < NPL; ++pl)
+      sx[f * NPL + pl] = *reinterpret_cast<const u32x4_t*>(kbase + at + ((pl * RB + srow + e) * 4 + f) * 1024 + 16 * lane);
+  };
+  auto sum_add = [&](int f) {
+#pragma unroll
+    for (int pl = 0; pl < NPL; ++pl) ssum[f & 1] = bf8_sum(sx[f * NPL + pl], f < 2 && pl == 0 ? 0.f : ssum[f & 1]);
+  };
+  auto fold = [&](int v, int f, float scale) {  // a quarter of block v's sum
+#pragma unroll
+    for (int r = 4 * f; r < 4 * f + 4; ++r)
+      acc[v % NB][v / NB][r] = fmaf(scale, au[v & 1][r], acc[v % NB][v / NB][r]);
+  };
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+#pragma unroll
+    for (int j = 0; j < PW; ++j) issue(s, s * STAGE, j);
+  if constexpr (EPI != DTREE_EPI_RESIDUAL) long_row_scale<T>(p, R, wave, rs);
+  stage_wait<(NST - 2) * PW>();
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): from here the compiler counts LDS operations alone
+#pragma unroll
+  for (int j = 0; j < NB; ++j) read_w(0, j);
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int pl = 0; pl < NPL; ++pl) read_a(0, 0, f, pl);
+#pragma unroll
+  for (int f = 0; f < 4; ++f) unpack(0, f);
+#pragma unroll
+  for (int j = 0; j < NB; ++j) sc[j] = 0.f;
+  float sc0 = __uint_as_float(sbw[0] << 16);  // column block 0's scale of the stage to come
+#pragma unroll
+  for (int r = 0; r < 16; ++r) au[(NT - 1) & 1][r] = 0.f;
+  // LDS offsets of stages s, s + 1 and s + NST - 1
+  unsigned cur = 0, nxt = STAGE, fut = (NST - 1) * STAGE;
+  auto advance = [](unsigned& o) { o = o + STAGE == NST * STAGE ? 0u : o + STAGE; };
+  for (int s = 0; s < S; ++s) {
+    const int slot = s & (kRing - 1);
+    const float last = sc[NB - 1];
+    sc[0] = sc0;
+#pragma unroll
+    for (int j = 1; j < NB; ++j) sc[j] = __uint_as_float(sbw[j] << 16);
+#pragma unroll
+    for (int e = 0; e < NCR; ++e)
+      cring[kg][min(wt * NCR + e, CB - 1) * 32 + c][slot] =
+          fmaf(-128.f, __uint_as_float(cw[e] << 16), __uint_as_float(cw[e] & 0xffff0000u));
+    // Block u = (row block i, column block j): its four MFMAs, with the previous
+    // block's fold, the unpacking of the column block needed next, the next
+    // row block's fragments, the ring's row sums and this stage's share of the
+    // loads between them.
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      const int i = u / NB, j = u % NB;
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        __builtin_amdgcn_sched_barrier(0);
+        // Inside the last row block: stage s + 1 has landed for every wave, every
+        // wave has read all of stage s, and the ring holds this group.
+        if (j == 0 && i + 1 == MB && f == 2) stage_wait<(NST - 3) * PW + PW * (NT - NB) / NT>();
+#pragma unroll
+        for (int pl = 0; pl < NPL; ++pl) {
+          if (f == 0 && pl == 0) {
+            f32x16_t z;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z[r] = 0.f;
+            au[u & 1] = mfma32(fa[0], bq[j][0], z);
+          } else {
+            au[u & 1] = mfma32(fa[f * NPL + pl], bq[j][f], au[u & 1]);
+          }
+          if (j + 1 == NB) {  // the next row block's fragments take this one's registers
+            if (i + 1 < MB) read_a(cur, i + 1, f, pl);
+            else read_a(nxt, 0, f, pl);
+          }
+        }
+        if (u > 0) fold(u - 1, f, sc[(u - 1) % NB]);
+        else fold(NT - 1, f, last);  // the previous stage's last block
+        if (u + 1 < NB) unpack(u + 1, f);
+        if (u + 1 == NT) unpack(0, f);
+        if (u < 2 * NSUM) {
+          if (u % 2 == 0) sum_read(cur, u / 2, f);
+          else sum_add(f);
+          if (u % 2 == 1 && f == 3) xring[kg][(srow + u / 2) * 32 + c][slot] = half_pair_sum(ssum[0] + ssum[1]);
+        }
+        if (i + 1 == MB && j == 0 && f == 2) {
+#pragma unroll
+          for (int jj = 0; jj < NB; ++jj) read_w(nxt, jj);
+        }
+        if (f == 3) {
+#pragma unroll
+          for (int d = PW * u / NT; d < PW * (u + 1) / NT; ++d) issue(s + NST - 1, fut, d);
+        }
+      }
+    }
+    sc0 = __uint_as_float(sbw[0] << 16);
+    advance(cur);
+    advance(nxt);
+    advance(fut);
+    if (slot == kRing - 1 || s + 1 == S) {
+      // the ring's groups: acc += sum(x) (b - 128 s), three bf16 parts each
+      const int valid = slot + 1;
+      auto parts = [&](const float* row, u32x4_t (&o)[3]) {
+        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(row), b = *reinterpret_cast<const f32x4_t*>(row + 4);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = e < valid ? (e < 4 ? a[e & 3] : b[e & 3]) : 0.f;
+        split3(v, o[0], o[1], o[2]);
+      };
+      u32x4_t cp[NB][2];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        u32x4_t o[3];
+        parts(cring[kg][(wn * NB + j) * 32 + c], o);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          cp[j][0][e] = h ? o[1][e] : o[0][e];
+          cp[j][1][e] = h ? o[0][e] : o[2][e];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        u32x4_t o[3], x3;
+        parts(xring[kg][(wm * MB + i) * 32 + c], o);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x3[e] = h ? o[2][e] : o[0][e];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          acc[j][i] = mfma32(o[0], cp[j][0], acc[j][i]);  // hi hi + hi mid
+          acc[j][i] = mfma32(o[1], cp[j][0], acc[j][i]);  // mid hi + mid mid
+          acc[j][i] = mfma32(x3, cp[j][1], acc[j][i]);    // hi lo + lo hi
+        }
+      }
+      lds_barrier();  // the next group's entries overwrite the ring
+    }
+  }
+#pragma unroll
+  for (int f = 0; f < 4; ++f) fold(NT - 1, f, sc[NB - 1]);
+  long_finish<T, EPI>(p, acc, smem, rs, wave, R, N0, [&](auto& a, float* buf) {
+#pragma unroll
+    for (auto& aj : a)
+#pragma unroll
+      for (auto& blk : aj) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) buf[acc_row(r, h) * 36 + c] = blk[r];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4_t v = *reinterpret_cast<const f32x4_t*>(buf + c * 36 + 8 * q + 4 * h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) blk[4 * q + e] = v[e];
+        }
+      }
+  });
+}
+
+enum Mode { kBf16, kBf16Lo, kF16, kQ4, kQ4Lo };
+
+template <class T, int EPI, Mode M>
+void launch_kernel(const LongParams& p, hipStream_t st) {
+  if constexpr (M == kQ4) longq_kernel<T, EPI, 1><<<p.tiles, T::THREADS, 0, st>>>(p);
+  else if constexpr (M == kQ4Lo) longq_kernel<T, EPI, 2><<<p.tiles, T::THREADS, 0, st>>>(p);
+  else long_kernel<T, EPI, M == kF16, M == kBf16Lo ? 2 : 1><<<p.tiles, T::THREADS, 0, st>>>(p);
+}
+
+template <class T, Mode M>
 int launch_tile(LongParams p, int epi, hipStream_t st) {
   p.ntn = (p.n + T::TN - 1) / T::TN;
   const long long tiles = (long long)((p.rows + T::TM - 1) / T::TM) * p.ntn;
   DTREE_REQUIRE(tiles < (1LL << 31), "gemm_long: grid too large");
   p.tiles = (int)tiles;
   switch (epi) {
-    case DTREE_EPI_STORE_F32: long_kernel<T, DTREE_EPI_STORE_F32, H, NPL><<<p.tiles, T::THREADS, 0, st>>>(p); break;
+    case DTREE_EPI_STORE_F32: launch_kernel<T, DTREE_EPI_STORE_F32, M>(p, st); break;
     case DTREE_EPI_RESIDUAL:
-      if constexpr (T::TN <= 256) long_kernel<T, DTREE_EPI_RESIDUAL, H, NPL><<<p.tiles, T::THREADS, 0, st>>>(p);
+      if constexpr (T::TN <= 256) launch_kernel<T, DTREE_EPI_RESIDUAL, M>(p, st);
       break;
-    case DTREE_EPI_SWIGLU: long_kernel<T, DTREE_EPI_SWIGLU, H, NPL><<<p.tiles, T::THREADS, 0, st>>>(p); break;
-    default: long_kernel<T, DTREE_EPI_STORE_BF16, H, NPL><<<p.tiles, T::THREADS, 0, st>>>(p); break;
+    case DTREE_EPI_SWIGLU: launch_kernel<T, DTREE_EPI_SWIGLU, M>(p, st); break;
+    default: launch_kernel<T, DTREE_EPI_STORE_BF16, M>(p, st); break;
   }
   DTREE_LAUNCH_CHECK("gemm_long launch");
   return DTREE_OK;
 }
 
+using Q128x128lo = Tile<2, 2, 2, 2, 3>;      // with the low activation plane
+using Q128x128k = Tile<2, 2, 2, 2, 3, 2>;
+using Q128x256 = Tile<2, 2, 2, 4, 3>;
+using Q256x192 = Tile<2, 3, 4, 2, 3>;
+using Q256x256 = Tile<4, 2, 2, 4, 3>;
 using T128x128 = Tile<2, 2, 2, 2, 4>;      // bf16 weights
 using T128x128k = Tile<2, 2, 2, 2, 4, 2>;
 using T256x128 = Tile<2, 2, 4, 2, 6>;
@@ -419,20 +762,27 @@ using T256x384 = Tile<4, 3, 2, 4, 3>;
 // 201 / 209 / 243 / 186; 4096 rows, N 24576 K 4096: 950 / 827 / 775 / 699 /
 // 697 / 728. The two widest do not take the residual epilogue (its preloaded
 // rows would not fit their registers).
-enum { kT128x128, kT256x128, kT256x192, kT256x256, kT256x320, kT256x384, kTiles };
 struct TileCost { int tm, tn; float cost; };
+enum { kT128x128, kT256x128, kT256x192, kT256x256, kT256x320, kT256x384, kTiles };
 constexpr TileCost kTileCost[kTiles] = {{128, 128, 0.55f}, {256, 128, 0.75f}, {256, 192, 1.08f},
                                         {256, 256, 1.30f}, {256, 320, 1.62f}, {256, 384, 2.05f}};
+// The same for q4 weights (one or two K blocks per stage; 128 x 128 tiles need
+// an even number of them). us at 1024 rows (128x128 / 128x256 / 256x192 /
+// 256x256): N 2560 K 9728 106 / 191 / 248 / 339; N 12352 K 2560 141 / 115 / 149
+// / 101; N 24576 K 4096 315 / 277 / 243 / 296; 4096 rows, N 24576 K 4096: 1211
+// / 1093 / 982 / 953.
+enum { kQ128x128, kQ128x256, kQ256x192, kQ256x256, kQTiles };
+constexpr TileCost kQTileCost[kQTiles] = {{128, 128, 0.84f}, {128, 256, 1.42f}, {256, 192, 1.87f}, {256, 256, 2.40f}};
 
-int pick_tile(int rows, int n, int epi, int cus) {
-  int best = 0;
+// The first of `count` shapes from `from` on with the least rounds x cost.
+int pick_tile(const TileCost* cost, int from, int count, int rows, int n, int cus) {
+  int best = from;
   float bt = 0.f;
-  for (int i = 0; i < kTiles; ++i) {
-    if (i >= kT256x320 && epi == DTREE_EPI_RESIDUAL) break;
-    const TileCost& c = kTileCost[i];
+  for (int i = from; i < count; ++i) {
+    const TileCost& c = cost[i];
     const long long tiles = (long long)((rows + c.tm - 1) / c.tm) * ((n + c.tn - 1) / c.tn);
     const float t = (float)((tiles + cus - 1) / cus) * c.cost;
-    if (i == 0 || t < bt) {
+    if (i == from || t < bt) {
       best = i;
       bt = t;
     }
@@ -444,14 +794,24 @@ int pick_tile(int rows, int n, int epi, int cus) {
 
 int launch_long_dense(LongParams p, int epi, bool h16, int cus, hipStream_t st) {
   if (!h16)
-    return p.x_lo ? launch_tile<T128x128, false, 2>(p, epi, st) : launch_tile<T128x128, false, 1>(p, epi, st);
-  switch (pick_tile(p.rows, p.n, epi, cus)) {
-    case kT256x128: return launch_tile<T256x128, true, 1>(p, epi, st);
-    case kT256x192: return launch_tile<T256x192, true, 1>(p, epi, st);
-    case kT256x256: return launch_tile<T256x256, true, 1>(p, epi, st);
-    case kT256x320: return launch_tile<T256x320, true, 1>(p, epi, st);
-    case kT256x384: return launch_tile<T256x384, true, 1>(p, epi, st);
-    default: return launch_tile<T128x128k, true, 1>(p, epi, st);
+    return p.x_lo ? launch_tile<T128x128, kBf16Lo>(p, epi, st) : launch_tile<T128x128, kBf16>(p, epi, st);
+  switch (pick_tile(kTileCost, 0, epi == DTREE_EPI_RESIDUAL ? kT256x320 : kTiles, p.rows, p.n, cus)) {
+    case kT256x128: return launch_tile<T256x128, kF16>(p, epi, st);
+    case kT256x192: return launch_tile<T256x192, kF16>(p, epi, st);
+    case kT256x256: return launch_tile<T256x256, kF16>(p, epi, st);
+    case kT256x320: return launch_tile<T256x320, kF16>(p, epi, st);
+    case kT256x384: return launch_tile<T256x384, kF16>(p, epi, st);
+    default: return launch_tile<T128x128k, kF16>(p, epi, st);
+  }
+}
+
+int launch_long_q4(LongParams p, int epi, int cus, hipStream_t st) {
+  if (p.x_lo) return launch_tile<Q128x128lo, kQ4Lo>(p, epi, st);
+  switch (pick_tile(kQTileCost, p.k % 128 ? kQ128x256 : kQ128x128, kQTiles, p.rows, p.n, cus)) {
+    case kQ128x256: return launch_tile<Q128x256, kQ4>(p, epi, st);
+    case kQ256x192: return launch_tile<Q256x192, kQ4>(p, epi, st);
+    case kQ256x256: return launch_tile<Q256x256, kQ4>(p, epi, st);
+    default: return launch_tile<Q128x128k, kQ4>(p, epi, st);
   }
 }
 

@@ -12,7 +12,7 @@ import pytest
 import torch
 
 from dtree_hip import _native as N
-from dtree_hip.weights import tile_weight_f16, untile_weight
+from dtree_hip.weights import q4_dequant, q4_random_mlx, q4_to_tiled, Q4Linear, tile_weight, tile_weight_f16, untile_weight
 
 pytestmark = pytest.mark.gpu
 
@@ -106,3 +106,47 @@ def test_long_tiles_64_column_tail(gpu_device, rows, n):
 @pytest.mark.parametrize("epi", [N.EPI_STORE_F32, N.EPI_RESIDUAL, N.EPI_SWIGLU, N.EPI_STORE_BF16])
 def test_long_tiles_misaligned_outputs(gpu_device, rows, n, epi):
     _long(gpu_device, rows, n, 128, epi, misaligned=True)
+
+
+# 128x128 (K halves), 128x256 (k % 128 != 0 or wide), 256x192, 256x256 tiles; a
+# K of 5, 8 and 19 groups ends inside, at and past the eight groups of a
+# correction step
+Q4_SHAPES = [(128, 256, 640), (128, 512, 512), (384, 19456, 320), (640, 19520, 576), (1152, 12352, 512),
+             (1152, 12352, 1216), (256, 320, 1216)]
+
+
+@pytest.mark.parametrize("rows,n,k", Q4_SHAPES)
+@pytest.mark.parametrize("lo", [False, True])
+def test_long_q4_tiles_match_float64(gpu_device, rows, n, k, lo):
+    """fp32 store; weights with a constant-group (scale 0) row block and a group
+    whose bias dwarfs its scale. The group sums are exact products of bf16
+    values accumulated in fp32 and the bias term carries 24 bits, so the error
+    stays within k 2^-23 of sum |x| (|s| 143 + |b|)."""
+    g = torch.Generator(device=gpu_device)
+    g.manual_seed(rows + n + k)
+    wq, sc, bi = q4_random_mlx(n, k, g, gpu_device)
+    sc[:32, 0] = 0.0
+    bi[32:64, 1] = 40.0
+    lin = Q4Linear(*q4_to_tiled(wq, sc, bi))
+    xf = torch.empty(rows, k, device=gpu_device).normal_(generator=g)
+    hi = xf.to(torch.bfloat16)
+    low = (xf - hi.float()).to(torch.bfloat16)
+    xt, xlt = tile_weight(hi), tile_weight(low)
+    ss = torch.rand(rows // 32, k // 32, 32, device=gpu_device, generator=g) + 0.5
+    out = torch.zeros(rows, n, device=gpu_device)
+    a = N.GemmArgs()
+    a.x = xt.data_ptr(); a.x_lo = xlt.data_ptr() if lo else None
+    a.x_layout = N.W_TILED; a.ldx = k; a.rows_padded = rows
+    a.w = lin.words.data_ptr(); a.w_scales = lin.sb.data_ptr(); a.w_layout = N.W_Q4G64; a.n = n; a.k = k
+    a.epilogue = N.EPI_STORE_F32; a.out_f32 = out.data_ptr(); a.ld_out_f32 = n
+    a.ss_in = ss.data_ptr(); a.ss_tiles = k // 32; a.norm_dim = k; a.eps = 1e-6
+    print(f"q4 gemm_long rows={rows} n={n} k={k} lo={lo}", flush=True)
+    N.check(N.lib().dtree_gemm_long(C.byref(a), torch.cuda.current_stream().cuda_stream), "gemm_long")
+    torch.cuda.synchronize()
+    rs = torch.rsqrt(ss.double().transpose(1, 2).reshape(rows, -1).sum(1) / k + 1e-6)
+    x = hi.double() + (low.double() if lo else 0.0)
+    ref = (x @ q4_dequant(lin).double().T) * rs[:, None]
+    mag = (x.abs() @ (143.0 * sc.double().abs() + bi.double().abs()).repeat_interleave(64, 1).T) * rs[:, None]
+    assert ((out.double() - ref).abs() <= k * 2.0 ** -23 * mag).all()
+    rel = ((out.double() - ref).norm() / ref.norm()).item()
+    assert rel <= 2e-6, rel  # fp32 sums: measured 3e-7
