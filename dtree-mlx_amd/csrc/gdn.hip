@@ -1610,29 +1610,34 @@ __global__ __launch_bounds__(256) void gdn_gated_norm_kernel(const DtreeStepDesc
 // the old window.
 constexpr int kChainAhead = 8;
 
+__device__ __forceinline__ void chain_window(int T, const float* __restrict__ x, int ldx, float* window, int C, int keep,
+                                             int first_block) {
+  const int c = ((int)blockIdx.x - first_block) * 256 + threadIdx.x;
+  if (c >= C) return;
+  float old[kConvMaxKeep];
+#pragma unroll
+  for (int r = 0; r < kConvMaxKeep; ++r) old[r] = r < keep ? window[(size_t)r * C + c] : 0.f;
+#pragma unroll
+  for (int r = 0; r < kConvMaxKeep; ++r) {
+    if (r >= keep) break;
+    // row r of the new window = element T + r of (old window ++ x)
+    const int e = T + r;
+    float val = 0.f;
+    if (e < keep) {
+#pragma unroll
+      for (int j = 0; j < kConvMaxKeep; ++j) val = j == e ? old[j] : val;
+    } else {
+      val = x[(size_t)(e - keep) * ldx + c];
+    }
+    window[(size_t)r * C + c] = val;
+  }
+}
+
 __global__ __launch_bounds__(256) void gdn_chain_scan_kernel(GdnParams p, const float* __restrict__ x, int ldx,
                                                              float* window, int C, int keep, int state_blocks) {
   const int T = p.T;
   if ((int)blockIdx.x >= state_blocks) {
-    const int c = ((int)blockIdx.x - state_blocks) * 256 + threadIdx.x;
-    if (c >= C) return;
-    float old[kConvMaxKeep];
-#pragma unroll
-    for (int r = 0; r < kConvMaxKeep; ++r) old[r] = r < keep ? window[(size_t)r * C + c] : 0.f;
-#pragma unroll
-    for (int r = 0; r < kConvMaxKeep; ++r) {
-      if (r >= keep) break;
-      // row r of the new window = element T + r of (old window ++ x)
-      const int e = T + r;
-      float val = 0.f;
-      if (e < keep) {
-#pragma unroll
-        for (int j = 0; j < kConvMaxKeep; ++j) val = j == e ? old[j] : val;
-      } else {
-        val = x[(size_t)(e - keep) * ldx + c];
-      }
-      window[(size_t)r * C + c] = val;
-    }
+    chain_window(T, x, ldx, window, C, keep, state_blocks);
     return;
   }
   constexpr int DK = 128, RPW = 8, A = kChainAhead;
@@ -1674,6 +1679,337 @@ __global__ __launch_bounds__(256) void gdn_chain_scan_kernel(GdnParams p, const 
     }
   }
   *reinterpret_cast<f32x4_t*>(sp) = s;
+}
+
+// ---- the chain in matrix form, 32 tokens at a time ------------------------------
+// (More than 40 tokens; the scan above for fewer.) Unrolled over a chunk of 32 tokens from its first state S_0 (the tree's matrix
+// form with parent t - 1), the recurrence is
+//   Delta = A (V - diag(gamma) K S_0^T),   A = (I + L)^-1 diag(beta),
+//   Y = diag(gamma) Q S_0^T + U Delta,     S_1 = gamma_31 S_0 + (diag(suf) Delta)^T K,
+// with gamma_t and suf_t the products of g over the chunk up to t and past t,
+// L[t][a] = beta_t D[t][a] (k_a . k_t) for a < t, U[t][a] = D[t][a] (k_a . q_t)
+// for a <= t, D[t][a] the product of g over (a, t]. A and U do not depend on
+// the state: gdn_chain_gram_kernel makes them for every chunk at once, and
+// gdn_chain_chunk_kernel walks the chunks with 72 MFMAs per wave and one
+// barrier per chunk where gdn_chain_scan_kernel makes 32 dependent steps.
+// (I + L)^-1 is a forward substitution over its two diagonal 16 x 16 blocks, one
+// column per lane, and two products for the third block: the products of
+// squarings that the shallow trees use would lose digits here, since on long
+// runs of similar keys the powers of L grow like binomials while the inverse
+// stays bounded. Products of g are formed directly, so g = 0 is no special case.
+//
+// The 64 floats per (token, value head) of A and U rows live in the layer's
+// `out` buffer between the two launches (128 16-bit values per head and token;
+// the gated norm overwrites all of it after). Rows: A [32] then U [32]; the
+// upper right quarters, which are zero and never read as matrix, hold gamma
+// (of A: rows 0 and 1, tokens 0-15 and 16-31) and suf (of U).
+constexpr int kChainChunk = 32;
+struct ChainScratch {
+  float* base;
+  size_t chunk, head, row;  // strides in floats
+};
+
+__global__ __launch_bounds__(256) void gdn_chain_gram_kernel(GdnParams p, ChainScratch sc) {
+  constexpr int DK = 128, LS = DK + 4, C = kChainChunk;
+  __shared__ __align__(16) float kq[2][C][LS];
+  __shared__ float gk[C][kMS], gq[C][kMS];
+  __shared__ __align__(16) float lu[4][2][C][kMS];  // per wave: L, U
+  __shared__ float sg[4][C], sb[4][2][C];
+  const int hk = blockIdx.x, chunk = blockIdx.y, t0 = chunk * C;
+  const int valid = min(C, p.T - t0);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {  // 2 x 32 rows x 32 float4
+    const int e = tid + 256 * i, m = e >> 10, t = (e >> 5) & 31, c = e & 31;
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+    if (t < valid) v = *reinterpret_cast<const f32x4_t*>((m ? p.q : p.k) + ((size_t)(t0 + t) * p.Hk + hk) * DK + 4 * c);
+    *reinterpret_cast<f32x4_t*>(&kq[m][t][4 * c]) = v;
+  }
+  __syncthreads();
+  {
+    const int bm = 16 * (wave >> 1), bn = 16 * (wave & 1);
+    const float* const A[2] = {&kq[0][bm][0], &kq[1][bm][0]};
+    const float* const B[2] = {&kq[0][bn][0], &kq[0][bn][0]};
+    f32x4_t acc[2];
+    tile16_dot_n<LS, DK / 16, 2>(A, B, lane, acc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      gk[bm + 4 * (lane >> 4) + i][bn + (lane & 15)] = acc[0][i];
+      gq[bm + 4 * (lane >> 4) + i][bn + (lane & 15)] = acc[1][i];
+    }
+  }
+  __syncthreads();
+  // One wave per value head of the group. Lane a of the first half runs down
+  // column a of L, of the second half down column a of U.
+  const int grp = p.Hv / p.Hk, a = lane & 31, half = lane >> 5;
+  for (int hh = wave; hh < grp; hh += 4) {
+    const int h = hk * grp + hh;
+    float* out = sc.base + chunk * sc.chunk + h * sc.head;
+    const bool live = a < valid;
+    const float beta = live ? p.beta[(size_t)(t0 + a) * p.Hv + h] : 0.f;
+    sg[wave][a] = live ? p.g[(size_t)(t0 + a) * p.Hv + h] : 1.f;
+    sb[wave][half][a] = half ? 1.f : beta;
+    const float* gram = half ? &gq[0][a] : &gk[0][a];
+    float d = 1.f, gamma = 1.f;  // D[t][a]; the product up to token a
+#pragma unroll
+    for (int t = 0; t < C; ++t) {
+      const float g = sg[wave][t];
+      d *= t > a ? g : 1.f;
+      gamma *= t <= a ? g : 1.f;
+      lu[wave][half][t][a] = t + half > a ? sb[wave][half][t] * d * gram[t * kMS] : 0.f;
+    }
+    if ((a >> 4) < valid) out[(a >> 4) * sc.row + 32 * half + 16 + (a & 15)] = half ? d : gamma;
+    // U, two rows per step (but the quarter that holds suf)
+#pragma unroll
+    for (int t = 0; t < C; t += 2)
+      if (t + half < valid && (t >= 16 || a < 16)) out[(t + half) * sc.row + 32 + a] = lu[wave][1][t + half][a];
+    // The diagonal 16 x 16 blocks of (I + L)^-1 by forward substitution: column
+    // c of block blk in lane 16 blk + c (twice, once per half-wave).
+    const int c = lane & 15, blk = a >> 4, kk = lane >> 4;
+    const float(*l)[kMS] = lu[wave][0];
+    float n[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      float s0 = t == c ? 1.f : 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
+#pragma unroll
+      for (int b = 0; b < t; b += 4) {
+        const f32x4_t lr = *reinterpret_cast<const f32x4_t*>(&l[16 * blk + t][16 * blk + b]);  // zero from t on
+        s0 = fmaf(-lr[0], n[b], s0);
+        if (b + 1 < t) s1 = fmaf(-lr[1], n[b + 1], s1);
+        if (b + 2 < t) s2 = fmaf(-lr[2], n[b + 2], s2);
+        if (b + 3 < t) s3 = fmaf(-lr[3], n[b + 3], s3);
+      }
+      n[t] = (s0 + s1) + (s2 + s3);
+    }
+    // into U's place in LDS: row-major, block blk's columns from 16 blk
+    float(*nv)[kMS] = lu[wave][1];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) nv[t][a] = n[t];
+    // the lower left block: -N22 (L21 N11); a product's accumulators are the
+    // next one's B operand (lane: column l % 16, rows 4 (l / 16) + i)
+    const float bc = sb[wave][0][c];
+    f32x4_t pr = {0.f, 0.f, 0.f, 0.f}, n21 = pr;
+    const f32x4_t l21 = *reinterpret_cast<const f32x4_t*>(&l[16 + c][4 * kk]);
+    const f32x4_t n22 = *reinterpret_cast<const f32x4_t*>(&nv[c][16 + 4 * kk]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pr = mfma16_f32(l21[i], nv[4 * kk + i][c], pr);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) n21 = mfma16_f32(n22[i], pr[i], n21);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = 4 * kk + i;
+      if (t < valid) out[t * sc.row + c] = nv[t][c] * bc;
+      if (16 + t < valid) {
+        out[(16 + t) * sc.row + c] = -n21[i] * bc;
+        out[(16 + t) * sc.row + 16 + c] = nv[t][16 + c] * sb[wave][0][16 + c];
+      }
+    }
+  }
+}
+
+// One workgroup per (value head, 16 value rows), four waves of 32 key dims
+// each; the transposed state slice stays in registers in the accumulator layout,
+// which is also the layout of an MFMA's B operand, so S_0 K^T, Delta and the
+// state update chain through registers. Only the four waves' partial K S_0^T
+// and Q S_0^T meet in LDS. A chunk's rows are staged in LDS two chunks ahead
+// (loading each wave's operands straight from memory instead took 41 loads per
+// wave and chunk and was bound by their issue: 2.6 us per chunk). The workgroups
+// of a key head run on one XCD. Workgroups past state_blocks advance the conv
+// window as in gdn_chain_scan_kernel.
+//
+// Bound by the serial chain of a chunk: 68 MFMAs of a wave (15 ns each), the
+// exchange and the operand reads, 2.5 us together. 1024 tokens of the
+// Qwen3.5-4B shape: 79 us for this launch and 14 for the chunk matrices, 385 us
+// token by token; the layer's core 421 -> 129 us.
+struct ChainOps {
+  f32x4_t k[2][2], q[2][2];  // [token tile][dim tile]: token 16 m + n, dims 4 kk ..
+  float kt[2][2][4];         // [dim tile][token tile]: dim n, tokens 4 kk ..
+  f32x4_t a[3], u[2];        // A (0,0), (1,0), (1,1); U (m, 0), (m, 1) of the wave's y tile
+  float v[2][4];             // token 16 m + 4 kk + i, value row n
+  f32x4_t gam[2], suf[2];
+};
+
+__global__ __launch_bounds__(256, 1) void gdn_chain_chunk_kernel(GdnParams p, ChainScratch sc, const float* x, int ldx,
+                                                              float* window, int C, int keep, int state_blocks) {
+  if ((int)blockIdx.x >= state_blocks) {
+    chain_window(p.T, x, ldx, window, C, keep, state_blocks);
+    return;
+  }
+  constexpr int DK = 128, R = 16, CH = kChainChunk;
+  __shared__ __align__(16) f32x4_t part[2][4][4][64];  // [parity][wave][k0 k1 q0 q1][lane]
+  struct Stage {  // a chunk's k and q rows, A | U rows and value columns
+    float k[CH][DK + 4], q[CH][DK + 4], m[CH][68], v[CH][20];
+  };
+  __shared__ __align__(16) Stage stg[2];
+  const int nsl = p.Dv / R;
+  // blocks of one key head share blockIdx % 8 when the key heads divide evenly
+  int b = blockIdx.x;
+  if (state_blocks % 8 == 0 && p.Hk % 8 == 0) b = (b & 7) * (state_blocks >> 3) + (b >> 3);
+  const int h = b / nsl, r0 = (b % nsl) * R, hk = h / (p.Hv / p.Hk);
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int d0 = 32 * wave, ym = wave & 1;
+  float* sp = p.state + ((size_t)h * p.Dv + r0 + n) * DK + d0 + 4 * kk;
+  f32x4_t s[2] = {*reinterpret_cast<const f32x4_t*>(sp), *reinterpret_cast<const f32x4_t*>(sp + 16)};
+  const int nch = (p.T + CH - 1) / CH;
+  const unsigned krow = (unsigned)p.Hk * DK * 4u, vrow = (unsigned)(p.Hv * p.Dv) * 4u, srow = (unsigned)sc.row * 4u;
+  // Loads of chunk c, ranged to its tokens: rows past them read as zero. They
+  // are issued on every path, also past the last chunk, so the compiler waits
+  // for one chunk's loads with the next one's in flight.
+  f32x4_t st_kq[8], st_m[2], st_v;
+  auto fetch = [&](int c) {
+    const int t0 = min(c, nch) * CH, valid = min(CH, p.T - t0);  // (chunk nch: nothing)
+    const unsigned some = valid > 0 ? ~0u : 0u;
+    const __amdgpu_buffer_rsrc_t kr = buf_rsrc(p.k + ((size_t)t0 * p.Hk + hk) * DK, ((valid - 1) * krow + DK * 4u) & some);
+    const __amdgpu_buffer_rsrc_t qr = buf_rsrc(p.q + ((size_t)t0 * p.Hk + hk) * DK, ((valid - 1) * krow + DK * 4u) & some);
+    const __amdgpu_buffer_rsrc_t vr =
+        buf_rsrc(p.v + ((size_t)t0 * p.Hv + h) * p.Dv, ((valid - 1) * vrow + p.Dv * 4u) & some);
+    const __amdgpu_buffer_rsrc_t sr =
+        buf_rsrc(sc.base + (t0 / CH) * sc.chunk + h * sc.head, ((valid - 1) * srow + 256u) & some);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // 32 rows of 32 float4
+      const unsigned off = (tid / 32 + 8 * i) * krow + 16u * (tid % 32);
+      st_kq[i] = __builtin_bit_cast(f32x4_t, buf_ld(kr, off));
+      st_kq[4 + i] = __builtin_bit_cast(f32x4_t, buf_ld(qr, off));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)  // 32 rows of 16
+      st_m[i] = __builtin_bit_cast(f32x4_t, buf_ld(sr, (tid / 16 + 16 * i) * srow + 16u * (tid % 16)));
+    // 32 rows of 16 floats (two threads each, the same value)
+    const int vt = (tid & 127) >> 2;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) st_v[i] = buf_ldf(vr, vt * vrow + (r0 + 4 * (tid & 3) + i) * 4u);
+  };
+  auto stage = [&](int c) {
+    Stage& b = stg[c & 1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      *reinterpret_cast<f32x4_t*>(&b.k[tid / 32 + 8 * i][4 * (tid % 32)]) = st_kq[i];
+      *reinterpret_cast<f32x4_t*>(&b.q[tid / 32 + 8 * i][4 * (tid % 32)]) = st_kq[4 + i];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) *reinterpret_cast<f32x4_t*>(&b.m[tid / 16 + 16 * i][4 * (tid % 16)]) = st_m[i];
+    *reinterpret_cast<f32x4_t*>(&b.v[(tid & 127) >> 2][4 * (tid & 3)]) = st_v;
+  };
+  auto read = [&](ChainOps& o, int c) {
+    const Stage& b = stg[c & 1];
+    auto f4 = [](const float* q) { return *reinterpret_cast<const f32x4_t*>(q); };
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        o.k[m][d] = f4(&b.k[16 * m + n][d0 + 16 * d + 4 * kk]);
+        o.q[m][d] = f4(&b.q[16 * m + n][d0 + 16 * d + 4 * kk]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o.kt[d][m][i] = b.k[16 * m + 4 * kk + i][d0 + 16 * d + n];
+      }
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      o.gam[m] = f4(&b.m[m][16 + 4 * kk]);
+      o.suf[m] = f4(&b.m[m][48 + 4 * kk]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o.v[m][i] = b.v[16 * m + 4 * kk + i][n];
+    }
+    o.a[0] = f4(&b.m[n][4 * kk]);
+    o.a[1] = f4(&b.m[16 + n][4 * kk]);
+    o.a[2] = f4(&b.m[16 + n][16 + 4 * kk]);
+    o.u[0] = f4(&b.m[16 * ym + n][32 + 4 * kk]);
+    o.u[1] = f4(&b.m[16 * ym + n][48 + 4 * kk]);
+  };
+  // Chunk c from o. After its barrier every wave has read chunk c's stage and
+  // chunk c + 1's is complete: the next operands come from there, and chunk
+  // c + 2 takes chunk c's place.
+  auto run = [&](const ChainOps& o, ChainOps& next, int c) {
+    const int t0 = c * CH, par = c & 1;
+    f32x4_t ks[2], qs[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) ks[m] = qs[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) ks[m] = mfma16_f32(o.k[m][d][i], s[d][i], ks[m]);
+#pragma unroll
+    for (int m = 0; m < 2; ++m) part[par][wave][m][lane] = ks[m];
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) qs[m] = mfma16_f32(o.q[m][d][i], s[d][i], qs[m]);
+#pragma unroll
+    for (int m = 0; m < 2; ++m) part[par][wave][2 + m][lane] = qs[m];
+    lds_barrier();  // (two parities: the next chunk's partials need no second one)
+    f32x4_t x2[2], dl[2], pk[2][4];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) pk[m][w] = part[par][w][m][lane];
+    __builtin_amdgcn_sched_barrier(0);  // all eight reads before the first sum
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const f32x4_t t = (pk[m][0] + pk[m][1]) + (pk[m][2] + pk[m][3]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x2[m][i] = o.v[m][i] - o.gam[m][i] * t[i];
+      dl[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      dl[0] = mfma16_f32(o.a[0][i], x2[0][i], dl[0]);
+      dl[1] = mfma16_f32(o.a[1][i], x2[0][i], dl[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dl[1] = mfma16_f32(o.a[2][i], x2[1][i], dl[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    read(next, c + 1);
+    stage(c + 2);
+    fetch(c + 3);
+    __builtin_amdgcn_sched_barrier(0);
+    // gamma_31 (tokens past the prompt have g = 1) = g_0 suf_0, lane 0's values
+    const float g31 = t0 >= p.T ? 1.f : __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, o.gam[0][0]))) *
+                      __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, o.suf[0][0])));
+#pragma unroll
+    for (int d = 0; d < 2; ++d) s[d] *= g31;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int d = 0; d < 2; ++d) s[d] = mfma16_f32(o.kt[d][m][i], dl[m][i] * o.suf[m][i], s[d]);
+    // y of token tile ym (waves 0 and 1 store it; ranged stores, the same count
+    // in every wave and chunk)
+    const int valid = min(CH, p.T - t0);
+    const __amdgpu_buffer_rsrc_t yr =
+        buf_rsrc(p.y + ((size_t)min(t0, p.T) * p.Hv + h) * p.Dv,
+                 valid > 0 && wave < 2 ? (unsigned)(valid - 1) * vrow + p.Dv * 4u : 0u);
+    f32x4_t y = part[par][0][2 + ym][lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) y += part[par][w][2 + ym][lane];
+    y *= ym ? o.gam[1] : o.gam[0];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y = mfma16_f32(o.u[0][i], dl[0][i], y);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y = mfma16_f32(o.u[1][i], ym ? dl[1][i] : 0.f, y);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, (float)y[i]), yr,
+                                            (int)((16 * ym + 4 * kk + i) * vrow + (r0 + n) * 4u), 0, 0);
+  };
+  ChainOps o0, o1;
+  fetch(0);
+  stage(0);
+  fetch(1);
+  lds_barrier();
+  read(o0, 0);
+  stage(1);
+  fetch(2);
+  for (int c = 0; c < nch; c += 2) {
+    run(o0, o1, c);
+    run(o1, o0, c + 1);  // (past the last chunk: no effect)
+  }
+  *reinterpret_cast<f32x4_t*>(sp) = s[0];
+  *reinterpret_cast<f32x4_t*>(sp + 16) = s[1];
 }
 
 // Rows per workgroup: the largest power of two <= 256 / (Dk / 4) and <= Dv
@@ -2110,9 +2446,27 @@ extern "C" int dtree_gdn_layer_chain(const DtreeGdnArgs* a, int32_t num_tokens, 
   p.T = num_tokens; p.Hk = a->num_k_heads; p.Hv = a->num_v_heads; p.Dv = a->head_v_dim; p.y = a->y;
   const int state_blocks = a->num_v_heads * (a->head_v_dim / 8);
   const int conv_blocks = (C + 255) / 256;
-  gdn_chain_scan_kernel<<<state_blocks + conv_blocks, 256, 0, stream>>>(p, a->proj, a->ld_proj, a->window, C,
-                                                                         a->conv_keep, state_blocks);
-  DTREE_LAUNCH_CHECK("gdn_layer_chain scan launch");
+  // Token by token up to 40 tokens (32: 31 us the layer's core, in matrix form 34;
+  // 64: 45 and 35; 1024: 421 and 129).
+  if (num_tokens <= 40) {
+    gdn_chain_scan_kernel<<<state_blocks + conv_blocks, 256, 0, stream>>>(p, a->proj, a->ld_proj, a->window, C,
+                                                                           a->conv_keep, state_blocks);
+    DTREE_LAUNCH_CHECK("gdn_layer_chain scan launch");
+  } else {
+    const bool rowmajor = a->out_layout == DTREE_W_ROWMAJOR;
+    ChainScratch sc;
+    sc.base = reinterpret_cast<float*>(a->out);
+    sc.row = rowmajor ? a->ld_out / 2 : 64;
+    sc.head = rowmajor ? 64 : (size_t)kChainChunk * 64;
+    sc.chunk = rowmajor ? kChainChunk * sc.row : (size_t)kChainChunk * 64 * a->num_v_heads;
+    const int chunks = (num_tokens + kChainChunk - 1) / kChainChunk;
+    gdn_chain_gram_kernel<<<dim3(a->num_k_heads, chunks), 256, 0, stream>>>(p, sc);
+    DTREE_LAUNCH_CHECK("gdn_layer_chain chunk matrices launch");
+    const int blocks = a->num_v_heads * (a->head_v_dim / 16);
+    gdn_chain_chunk_kernel<<<blocks + conv_blocks, 256, 0, stream>>>(p, sc, a->proj, a->ld_proj, a->window, C,
+                                                                     a->conv_keep, blocks);
+    DTREE_LAUNCH_CHECK("gdn_layer_chain chunk launch");
+  }
   const int pairs = a->rows_padded * a->num_v_heads;
   const int per_block = 256 / (128 / 8);
   gdn_gated_norm_kernel<128><<<(pairs + per_block - 1) / per_block, 256, 0, stream>>>(
