@@ -313,29 +313,27 @@ class TreeEngineBase:
         a.rows_padded = rows
         N.check(self.lib.dtree_gemm_long(C.byref(a), st), f"long gemm {name}")
 
-    def _prefill_chunks(self, pf: dict, P0: int, n: int, rows: int, rope_dims: int, st: int) -> int:
-        """Step descriptors of a segment's 128-row causal chunks (chain trees
-        over the cached prefix: chunk ch holds positions P0 + 128 ch ..) and
-        their RoPE tables over rope_dims dims; returns the descriptor stride."""
-        nch = rows // 128
-        recs = np.zeros(nch, dtype=N.STEP_DESC_DTYPE)
-        for ch in range(nch):
-            L = min(128, n - 128 * ch)
-            r = recs[ch]
-            r["past_length"] = P0 + 128 * ch
-            r["num_nodes"] = L
-            r["bonus_token"] = -1
-            r["positions"][:L] = np.arange(P0 + 128 * ch, P0 + 128 * ch + L)
-            r["parents"][:] = -1
-            r["parents"][1:L] = np.arange(L - 1)
-            r["ancestors"][:L] = ancestor_bitsets([-1] + list(range(L - 1)))
-        pf["descs"][:nch].copy_(torch.from_numpy(recs.view(np.uint8).reshape(nch, -1)))
-        dstride = pf["descs"].shape[1]
-        for ch in range(nch):
-            N.check(self.lib.dtree_rope_table(pf["descs"].data_ptr() + ch * dstride, 128, rope_dims,
-                                              self.cfg.rope_theta, pf["cos"][128 * ch].data_ptr(),
-                                              pf["sin"][128 * ch].data_ptr(), st), "rope table")
-        return dstride
+    def _prefill_rope(self, pf: dict, P0: int, rows: int, rope_dims: int, st: int) -> None:
+        """RoPE tables of a segment's rows (positions P0 ..) over rope_dims dims."""
+        N.check(self.lib.dtree_rope_positions(P0, rows, rope_dims, self.cfg.rope_theta, pf["cos"].data_ptr(),
+                                              pf["sin"].data_ptr(), st), "rope positions")
+
+    def _prefill_attention(self, pf: dict, lw, kv: PagedKVCache, slot: int, P0: int, n: int, rows: int, st: int,
+                           **geometry) -> None:
+        """Causal attention of a segment's n rows (appending their K / V) in one call."""
+        c = self.cfg
+        a = N.AttnArgs()
+        a.qkv = pf["qkv"].data_ptr(); a.ld_qkv = pf["qkv"].shape[1]
+        a.q_norm = lw.q_norm.data_ptr(); a.k_norm = lw.k_norm.data_ptr(); a.eps = c.rms_norm_eps
+        a.rope_cos = pf["cos"].data_ptr(); a.rope_sin = pf["sin"].data_ptr()
+        a.k_pages = kv.k_ptr(slot); a.v_pages = kv.v_ptr(slot); a.page_table = kv.page_table.data_ptr()
+        a.out = pf["attn"][0].data_ptr(); a.out_lo = self.lo_ptr(pf["attn"])
+        a.ld_out = c.q_dim; a.out_layout = self.w.layout
+        a.num_heads = c.num_attention_heads; a.num_kv_heads = c.num_key_value_heads; a.head_dim = c.head_dim
+        a.rows_padded = rows; a.scale = c.head_dim ** -0.5
+        for name, v in geometry.items():
+            setattr(a, name, v)
+        N.check(self.lib.dtree_causal_attention(C.byref(a), P0, n, st), "prefill attention")
 
     def _prefill_logits(self, pf: dict, n: int, st: int) -> torch.Tensor:
         """fp32 logits [1, 1, V] of a segment's last row (its xg / ss rows hold
@@ -719,19 +717,15 @@ class Qwen3TreeEngine(TreeEngineBase):
                   act=torch.zeros(2, rows, F, dtype=self.act_dtype, device=dev),
                   hidden=torch.zeros(rows, nh * H, dtype=bf16, device=dev),
                   cos=torch.zeros(rows, D // 2, dtype=f32, device=dev),
-                  sin=torch.zeros(rows, D // 2, dtype=f32, device=dev),
-                  descs=torch.zeros(rows // 128, C.sizeof(N.StepDesc), dtype=torch.uint8, device=dev),
-                  attn_ws=torch.zeros(self.lib.dtree_attention_workspace_bytes(c.num_attention_heads, D,
-                                                                               self.max_past, 128),
-                                      dtype=torch.uint8, device=dev))
+                  sin=torch.zeros(rows, D // 2, dtype=f32, device=dev))
         self._pf = pf
         return pf
 
     def prefill_long(self, cache: PagedKVCache, tokens, want_logits: bool = True):
         """Causal forward over the prompt with the long-M GEMM: per segment of
         up to PREFILL_SEGMENT tokens, embed, then per layer the fused QKV GEMM,
-        attention per 128-row chunk (a chain "tree" over the cached prefix,
-        appending its K/V rows), o_proj, gate/up and down_proj. Returns the
+        causal attention over the cached prefix and the segment (appending its
+        K/V rows), o_proj, gate/up and down_proj. Returns the
         fp32 logits of the last position ([1, 1, V]) if asked and the
         verifier hidden rows of every position ([n, n_ids * H] bf16 or None)."""
         if not self.supports_long_prefill():
@@ -757,34 +751,18 @@ class Qwen3TreeEngine(TreeEngineBase):
             pf = self._prefill_buffers(max(rows, seg if len(toks) > seg else rows))
             P0 = cache.offset
             pf["tokens"][:n].copy_(torch.tensor(part, dtype=torch.int32))
-            nch = rows // 128
             N.check(self.lib.dtree_embed_tokens(
                 pf["tokens"].data_ptr(), n, emb, emb_layout, emb_sb, c.vocab_size, H,
                 self.w.layers[0].input_norm.data_ptr(), rows, pf["x"].data_ptr(), pf["xg"][0].data_ptr(),
                 self.lo_ptr(pf["xg"]), self.w.layout, pf["ss"].data_ptr(), st), "embed tokens")
-            dstride = self._prefill_chunks(pf, P0, n, rows, D, st)
+            self._prefill_rope(pf, P0, rows, D, st)
             nL = c.num_hidden_layers
             for li in range(nL):
                 lw = self.w.layers[li]
                 nxt = self.w.layers[li + 1].input_norm if li + 1 < nL else self.w.final_norm
                 self._long_gemm("qkv", pf["xg"], H, lw.wqkv, N.EPI_STORE_F32, rows, st, ss_in=pf["ss"],
                                 out_f32=pf["qkv"])
-                for ch in range(nch):
-                    a = N.AttnArgs()
-                    a.qkv = pf["qkv"][128 * ch].data_ptr(); a.ld_qkv = c.qkv_dim
-                    a.q_norm = lw.q_norm.data_ptr(); a.k_norm = lw.k_norm.data_ptr(); a.eps = c.rms_norm_eps
-                    a.rope_cos = pf["cos"][128 * ch].data_ptr(); a.rope_sin = pf["sin"][128 * ch].data_ptr()
-                    a.k_pages = cache.k_ptr(li); a.v_pages = cache.v_ptr(li)
-                    a.page_table = cache.page_table.data_ptr()
-                    a.desc = pf["descs"].data_ptr() + ch * dstride
-                    a.out = pf["attn"][0, 128 * ch].data_ptr()
-                    a.out_lo = self.lo_ptr(pf["attn"], 2 * 128 * ch * c.q_dim)
-                    a.ld_out = c.q_dim; a.out_layout = self.w.layout
-                    a.num_heads = c.num_attention_heads; a.num_kv_heads = c.num_key_value_heads; a.head_dim = D
-                    a.rows_padded = 128; a.scale = D ** -0.5
-                    a.max_past_length = self.attn_grid_past(P0 + 128 * ch); a.write_cache = 1
-                    a.workspace = pf["attn_ws"].data_ptr(); a.workspace_bytes = pf["attn_ws"].numel()
-                    N.check(self.lib.dtree_tree_attention(C.byref(a), st), "prefill attention")
+                self._prefill_attention(pf, lw, cache, li, P0, n, rows, st)
                 self._long_gemm("o", pf["attn"], c.q_dim, lw.wo, N.EPI_RESIDUAL, rows, st, out_f32=pf["x"],
                                 out_bf16=pf["xg"], next_norm=lw.post_norm, ss_out=pf["ss"])
                 self._long_gemm("gu", pf["xg"], H, lw.wgu, N.EPI_SWIGLU, rows, st, ss_in=pf["ss"], out_bf16=pf["act"])
@@ -798,7 +776,6 @@ class Qwen3TreeEngine(TreeEngineBase):
             cache.offset = P0 + n
             if self.layer_ids:
                 hid_parts.append(pf["hidden"][:n].clone())
-        self.launch_attention_status(pf["attn_ws"], st)
         logits = self._prefill_logits(pf, n, st) if want_logits else None
         hidden = torch.cat(hid_parts, 0) if hid_parts else None
         return logits, hidden

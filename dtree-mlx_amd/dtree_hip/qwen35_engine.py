@@ -265,11 +265,7 @@ class Qwen35TreeEngine(TreeEngineBase):
                   act=torch.zeros(2, rows, F, dtype=self.act_dtype, device=dev),
                   hidden=torch.zeros(rows, nh * H, dtype=bf16, device=dev),
                   cos=torch.zeros(rows, c.rope_dims // 2, dtype=f32, device=dev),
-                  sin=torch.zeros(rows, c.rope_dims // 2, dtype=f32, device=dev),
-                  descs=torch.zeros(rows // 128, C.sizeof(N.StepDesc), dtype=torch.uint8, device=dev),
-                  attn_ws=torch.zeros(self.lib.dtree_attention_workspace_bytes(c.num_attention_heads, c.head_dim,
-                                                                               self.max_past, 128),
-                                      dtype=torch.uint8, device=dev))
+                  sin=torch.zeros(rows, c.rope_dims // 2, dtype=f32, device=dev))
         self._pf = pf
         return pf
 
@@ -299,14 +295,14 @@ class Qwen35TreeEngine(TreeEngineBase):
         PREFILL_SEGMENT tokens, embed, then per GatedDeltaNet layer the in_proj
         GEMM, the chain prep + recurrence + gated norm (dtree_gdn_layer_chain:
         the committed window and state advance over the segment) and out_proj;
-        per attention layer the fused QKV GEMM, gated attention per 128-row
-        chunk (appending its K/V rows) and o_proj; then the MLP. Returns the
+        per attention layer the fused QKV GEMM, causal gated attention
+        (appending its K/V rows) and o_proj; then the MLP. Returns the
         fp32 logits of the last position ([1, 1, V]) if asked and the verifier
         hidden rows of every position ([n, n_ids * H] bf16 or None)."""
         if not self.supports_long_prefill():
             raise NotImplementedError("the long-M prefill runs tiled weights")
         c = self.cfg
-        H, D = c.hidden_size, c.head_dim
+        H = c.hidden_size
         toks = [int(t) for t in tokens]
         if not toks:
             raise ValueError("empty prompt")
@@ -327,12 +323,11 @@ class Qwen35TreeEngine(TreeEngineBase):
             pf = self._prefill_buffers(max(rows, seg if len(toks) > seg else rows))
             P0 = cache.offset
             pf["tokens"][:n].copy_(torch.tensor(part, dtype=torch.int32))
-            nch = rows // 128
             N.check(self.lib.dtree_embed_tokens(
                 pf["tokens"].data_ptr(), n, emb, emb_layout, emb_sb, c.vocab_size, H,
                 self.w.layers[0].input_norm.data_ptr(), rows, pf["x"].data_ptr(), pf["xg"][0].data_ptr(),
                 self.lo_ptr(pf["xg"]), self.w.layout, pf["ss"].data_ptr(), st), "embed tokens")
-            dstride = self._prefill_chunks(pf, P0, n, rows, c.rope_dims, st)
+            self._prefill_rope(pf, P0, rows, c.rope_dims, st)
             nL = c.num_hidden_layers
             for li in range(nL):
                 lw = self.w.layers[li]
@@ -348,22 +343,7 @@ class Qwen35TreeEngine(TreeEngineBase):
                     ai = cache.slot[li]
                     self._long_gemm("qkv", pf["xg"], H, lw.wqkv, N.EPI_STORE_F32, rows, st, ss_in=pf["ss"],
                                     out_f32=pf["qkv"])
-                    for ch in range(nch):
-                        a = N.AttnArgs()
-                        a.qkv = pf["qkv"][128 * ch].data_ptr(); a.ld_qkv = c.attn_qkv_dim
-                        a.q_norm = lw.q_norm.data_ptr(); a.k_norm = lw.k_norm.data_ptr(); a.eps = c.rms_norm_eps
-                        a.rope_cos = pf["cos"][128 * ch].data_ptr(); a.rope_sin = pf["sin"][128 * ch].data_ptr()
-                        a.k_pages = kv.k_ptr(ai); a.v_pages = kv.v_ptr(ai); a.page_table = kv.page_table.data_ptr()
-                        a.desc = pf["descs"].data_ptr() + ch * dstride
-                        a.out = pf["attn"][0, 128 * ch].data_ptr()
-                        a.out_lo = self.lo_ptr(pf["attn"], 2 * 128 * ch * c.q_dim)
-                        a.ld_out = c.q_dim; a.out_layout = self.w.layout
-                        a.num_heads = c.num_attention_heads; a.num_kv_heads = c.num_key_value_heads
-                        a.head_dim = D; a.rows_padded = 128; a.scale = D ** -0.5
-                        a.max_past_length = self.attn_grid_past(P0 + 128 * ch); a.write_cache = 1
-                        a.workspace = pf["attn_ws"].data_ptr(); a.workspace_bytes = pf["attn_ws"].numel()
-                        a.rope_dims = c.rope_dims; a.gated = 1
-                        N.check(self.lib.dtree_tree_attention(C.byref(a), st), "prefill attention")
+                    self._prefill_attention(pf, lw, kv, ai, P0, n, rows, st, rope_dims=c.rope_dims, gated=1)
                     self._long_gemm("o", pf["attn"], c.q_dim, lw.wo, N.EPI_RESIDUAL, rows, st, out_f32=pf["x"],
                                     out_bf16=pf["xg"], next_norm=lw.post_norm, ss_out=pf["ss"])
                 self._long_gemm("gu", pf["xg"], H, lw.wgu, N.EPI_SWIGLU, rows, st, ss_in=pf["ss"],
@@ -378,7 +358,6 @@ class Qwen35TreeEngine(TreeEngineBase):
             cache.offset = P0 + n
             if self.layer_ids:
                 hid_parts.append(pf["hidden"][:n].clone())
-        self.launch_attention_status(pf["attn_ws"], st)
         logits = self._prefill_logits(pf, n, st) if want_logits else None
         hidden = torch.cat(hid_parts, 0) if hid_parts else None
         return logits, hidden

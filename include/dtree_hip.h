@@ -362,6 +362,23 @@ int dtree_embed_tokens(const int32_t* tokens, int32_t n, const uint16_t* embed, 
                        hipStream_t stream);
 
 /*
+ * Causal attention of a whole prompt segment (the attention of
+ * forward_with_hidden_states, adapters.py:494-533, over a cache that holds
+ * past_length positions): rows 0 .. num_rows - 1 of qkv are positions
+ * past_length + row; their K / V rows are appended to the cache (page_table
+ * covers past_length + num_rows positions) and row r attends to every position
+ * up to its own. Arguments as for dtree_tree_attention, with qkv, out and the
+ * RoPE tables of rows_padded rows (a multiple of 32; rows >= num_rows of out
+ * become zero); desc, max_past_length, write_cache and the workspace are not
+ * used. q_norm and the pages are 16-byte aligned. dtree_rope_positions fills
+ * such tables ([rows][rope_dims / 2]) for positions first_position + row, as
+ * dtree_rope_table does for a tree's positions.
+ */
+int dtree_causal_attention(const DtreeAttnArgs* args, int32_t past_length, int32_t num_rows, hipStream_t stream);
+int dtree_rope_positions(int32_t first_position, int32_t rows, int32_t rope_dims, float rope_base, float* rope_cos,
+                         float* rope_sin, hipStream_t stream);
+
+/*
  * Layer input from caller rows instead of token ids: the DFlash drafter's
  * noise embedding enters its first decoder layer (DFlashDraftModel.__call__,
  * draft.py:349-364, input_layernorm at draft.py:294-295). rows: bf16
