@@ -6,7 +6,8 @@
 //
 // Three launches, all graph-capturable:
 //   1. topk_chunk_kernel  (row, 8192-logit chunk): chunk max and sum of
-//      exp(x - max), and the chunk's top-k by a four-digit radix select;
+//      exp(x - max), and the chunk's top-k by a bound (bounded_topk) or, where
+//      that does not thin the chunk out, a four-digit radix select;
 //   2. topk_merge_kernel  (row): the union of the chunk candidates (which
 //      holds the row's top-k) selected the same way and sorted; log-probs
 //      from the merged logsumexp;
@@ -42,6 +43,19 @@ __device__ __forceinline__ uint32_t ordered_bits(float x) {
 }
 __device__ __forceinline__ float from_ordered(uint32_t o) {
   return __uint_as_float((o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
+}
+
+// Wave-wide unsigned maximum (in every lane) by the cross-lane adders of the
+// vector unit: six dependent operations, where shuffles go through LDS.
+__device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
+  auto step = [&](uint32_t o) { v = max(v, o); };
+  step(__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  step(__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1, 3
+  step(__builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2, 3
+  return __builtin_amdgcn_readlane(v, 63);
 }
 
 struct SelectLds {
@@ -171,6 +185,65 @@ __device__ void select_topk(const uint32_t (&hi)[E], const uint32_t (&lo)[E], co
   }
 }
 
+constexpr int kShort = 256;  // candidates that bounded_topk ranks
+struct ShortLds {
+  __attribute__((aligned(16))) uint32_t tmax[kThreads];
+  unsigned long long cand[kShort];
+  uint32_t bound, n;
+};
+
+// The same list by a bound: the K-th largest of the threads' own maxima is at
+// most the K-th largest element, so the elements from it on (about K of them
+// when the values are spread over the threads) hold the top K; they are
+// compacted, and each is placed by counting the larger ones. hi[e] of an
+// invalid element is 0. The maxima are compared by their upper 24 bits, then
+// by thread. False (same in every thread) if more than kShort elements reach the bound - many
+// equal values, or the largest ones in few threads - or if fewer than K threads
+// hold any: the radix select has to take over.
+template <int E>
+__device__ bool bounded_topk(const uint32_t (&hi)[E], const uint32_t (&lo)[E], int K, ShortLds& b,
+                             unsigned long long* list) {
+  const int t = threadIdx.x;
+  uint32_t m = 0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) m = max(m, hi[e]);
+  m = (m & ~255u) | (uint32_t)(255 - t);
+  b.tmax[t] = m;
+  if (t == 0) {
+    b.bound = 0;
+    b.n = 0;
+  }
+  __syncthreads();
+  int above = 0;
+#pragma unroll 8
+  for (int i = 0; i < kThreads; i += 4) {
+    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&b.tmax[i]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) above += v[j] > m ? 1 : 0;
+  }
+  if (above == K - 1) b.bound = m & ~255u;
+  __syncthreads();
+  const uint32_t bound = b.bound;
+  if (bound == 0) return false;
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (hi[e] >= bound) {
+      const uint32_t slot = atomicAdd(&b.n, 1u);
+      if (slot < (uint32_t)kShort) b.cand[slot] = ((unsigned long long)hi[e] << 32) | lo[e];
+    }
+  __syncthreads();
+  const int n = (int)b.n;
+  if (n > kShort) return false;
+  if (t < n) {
+    const unsigned long long key = b.cand[t];
+    int rank = 0;
+    for (int i = 0; i < n; ++i) rank += b.cand[i] > key ? 1 : 0;
+    if (rank < K) list[rank] = key;
+  }
+  __syncthreads();
+  return true;
+}
+
 __device__ __forceinline__ float block_max(float v, float* red) {
   const int t = threadIdx.x;
 #pragma unroll
@@ -207,8 +280,12 @@ struct TreeParams {
   float* topk_lp;
 };
 
+// Latency-bound. Measured, 15 rows of 151936 logits, top 24: 13.5 us by the
+// bound, 22.6 by the radix select alone (its first digit, sign and exponent,
+// puts most of 8192 histogram increments on a few LDS words).
 __global__ __launch_bounds__(kThreads) void topk_chunk_kernel(TreeParams p) {
   __shared__ SelectLds s;
+  __shared__ ShortLds b;
   __shared__ float red[kThreads / 64];
   const int row = blockIdx.y, chunk = blockIdx.x, t = threadIdx.x;
   const int base = chunk * kChunk + kE1 * t;
@@ -240,29 +317,31 @@ __global__ __launch_bounds__(kThreads) void topk_chunk_kernel(TreeParams p) {
   uint32_t hi[kE1], lo[kE1];
 #pragma unroll
   for (int e = 0; e < kE1; ++e) {
-    hi[e] = ordered_bits(x[e]);
+    hi[e] = valid[e] ? ordered_bits(x[e]) : 0u;
     lo[e] = ~(uint32_t)(base + e);  // smaller token id sorts first among equal logits
   }
-  select_topk<kE1>(hi, lo, valid, p.k, s);
+  if (!bounded_topk<kE1>(hi, lo, p.k, b, s.list)) select_topk<kE1>(hi, lo, valid, p.k, s);
   unsigned long long* dst = p.part_keys + ((size_t)row * p.chunks + chunk) * p.k;
   for (int i = t; i < p.k; i += kThreads) dst[i] = s.list[i];
 }
 
+// As above: 7.1 us for 15 rows of 19 x 24 candidates, 10.4 by the radix
+// select alone.
 __global__ __launch_bounds__(kThreads) void topk_merge_kernel(TreeParams p) {
   __shared__ SelectLds s;
+  __shared__ ShortLds b;
   __shared__ float red[kThreads / 64];
   const int row = blockIdx.x, t = threadIdx.x;
   const int n = p.chunks * p.k;
   const unsigned long long* src = p.part_keys + (size_t)row * n;
   uint32_t hi[kE2], lo[kE2];
-  bool valid[kE2];
+  // a chunk's candidates are sorted: neighbours go to different threads
 #pragma unroll
   for (int e = 0; e < kE2; ++e) {
-    const int i = kE2 * t + e;  // candidates of chunk c precede chunk c + 1's: position order = token id order
+    const int i = kThreads * e + t;
     const unsigned long long key = i < n ? src[i] : 0ull;
     hi[e] = (uint32_t)(key >> 32);
     lo[e] = (uint32_t)key;
-    valid[e] = key != 0ull;
   }
   // logsumexp of the row from the chunk partials
   float mm = -__builtin_inff();
@@ -275,7 +354,18 @@ __global__ __launch_bounds__(kThreads) void topk_merge_kernel(TreeParams p) {
   }
   ss = block_sum(ss, red);
   const float lse = mm + logf(ss);
-  select_topk<kE2>(hi, lo, valid, p.k, s);
+  if (!bounded_topk<kE2>(hi, lo, p.k, b, s.list)) {
+    bool valid[kE2];
+#pragma unroll
+    for (int e = 0; e < kE2; ++e) {
+      const int i = kE2 * t + e;  // candidates of chunk c precede chunk c + 1's: position order = token id order
+      const unsigned long long key = i < n ? src[i] : 0ull;
+      hi[e] = (uint32_t)(key >> 32);
+      lo[e] = (uint32_t)key;
+      valid[e] = key != 0ull;
+    }
+    select_topk<kE2>(hi, lo, valid, p.k, s);
+  }
   for (int i = t; i < p.k; i += kThreads) {
     const unsigned long long key = s.list[i];
     const int tok = (int)~(uint32_t)key;
@@ -296,110 +386,169 @@ __device__ __forceinline__ void add_level(unsigned long long& r0, unsigned long 
     r1 += v << (64 - 7 * (level - 9));
 }
 
-// (logw, r0, r1) a better heap entry than (lw, q0, q1)?
-__device__ __forceinline__ bool better(double logw, unsigned long long r0, unsigned long long r1, double lw,
-                                       unsigned long long q0, unsigned long long q1) {
-  if (logw != lw) return logw > lw;
-  if (r0 != q0) return r0 < q0;
-  return r1 < q1;
+// A heap entry's logw as an unsigned integer of the same order (NaN: the
+// smallest) and back.
+__device__ __forceinline__ unsigned long long ordered_key(double x) {
+  if (x != x) return 0ull;
+  const unsigned long long b = (unsigned long long)__double_as_longlong(x + 0.0);  // -0 compares as +0
+  return (b >> 63) ? ~b : (b | 1ull << 63);
+}
+__device__ __forceinline__ double key_logw(unsigned long long k) {
+  return __longlong_as_double((long long)((k >> 63) ? k & ~(1ull << 63) : ~k));
 }
 
+__device__ __forceinline__ unsigned long long readlane64(unsigned long long v, int lane) {
+  return ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), lane) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
+
+// One wavefront; a serial chain of `budget` pops. Everything a pop needs is in
+// registers (entry i of the heap in lane i % 64, slot i / 64 of ES; node i alike
+// in NS slots) or in LDS (the top-k lists); its winner is found by DPP maxima
+// over the keys' halves, and only equal keys go on to the ranks. Bound by the
+// instructions of a pop, hence the slot counts as template arguments. Measured,
+// 24 pops over 15 rows: 15 us with one slot, 24.4 with four; with the
+// entries in LDS, shuffles of (logw, ranks, index) and the lists read from
+// memory at every pop, 40 us.
+template <int ES, int NS>
 __global__ __launch_bounds__(64) void heap_kernel(TreeParams p) {
-  __shared__ double e_logw[kMaxEntries];
-  __shared__ unsigned long long e_r0[kMaxEntries], e_r1[kMaxEntries];
-  __shared__ int e_meta[kMaxEntries];  // parent | depth << 8 | rank << 16; -1 = popped
-  __shared__ int n_tok[DTREE_MAX_NODES], n_par[DTREE_MAX_NODES], n_dep[DTREE_MAX_NODES];
-  __shared__ uint32_t n_anc[DTREE_MAX_NODES][DTREE_MASK_WORDS];
+  constexpr int NW = 2 * NS;  // bitset words that NS slots of nodes use
+  static_assert(NW <= DTREE_MASK_WORDS && 64 * NS <= DTREE_MAX_NODES, "nodes of the descriptor");
+  __shared__ float s_lp[kMaxDepth * kMaxK];
+  __shared__ int s_tok[kMaxDepth * kMaxK];
   const int lane = threadIdx.x;
+  unsigned long long key[ES], r0[ES], r1[ES];
+  int meta[ES];  // parent | depth << 8 | rank << 16; -1 = no entry
+  int tok[NS], par[NS], dep[NS];
+  uint32_t anc[NS][NW];
+#pragma unroll
+  for (int s = 0; s < ES; ++s) {
+    key[s] = r0[s] = r1[s] = 0ull;
+    meta[s] = -1;
+  }
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    tok[s] = dep[s] = 0;
+    par[s] = -1;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) anc[s][w] = 0u;
+  }
+  if (lane == 0) {  // node 0, the root
+    tok[0] = p.root;
+    anc[0][0] = 1u;
+  }
   int n_ent = 0, nodes = 0;
   if (p.budget > 0 && p.depth > 0) {
+    const int n = p.depth * p.k;
+#pragma unroll 8
+    for (int i = lane; i < n; i += 64) {
+      s_lp[i] = p.top_lp[i];
+      s_tok[i] = p.top_tok[i];
+    }
+    __syncthreads();
     if (lane == 0) {
-      e_logw[0] = (double)p.top_lp[0];
-      e_r0[0] = 1ull << 57;  // ranks (0,)
-      e_r1[0] = 0ull;
-      e_meta[0] = 0 | (1 << 8) | (0 << 16);
+      key[0] = ordered_key((double)s_lp[0]);
+      r0[0] = 1ull << 57;  // ranks (0,)
+      meta[0] = 0 | (1 << 8) | (0 << 16);
     }
     n_ent = 1;
   }
-  __syncthreads();
   while (nodes < p.budget && n_ent > 0) {
-    double bl = -__builtin_inff();
-    unsigned long long b0 = ~0ull, b1 = ~0ull;
-    int bi = -1;
-    for (int i = lane; i < n_ent; i += 64) {
-      if (e_meta[i] < 0) continue;
-      if (bi < 0 || better(e_logw[i], e_r0[i], e_r1[i], bl, b0, b1)) {
-        bl = e_logw[i];
-        b0 = e_r0[i];
-        b1 = e_r1[i];
-        bi = i;
+    unsigned long long bk = key[0], b0 = r0[0], b1 = r1[0];
+    int bm = meta[0], bs = 0;
+#pragma unroll
+    for (int s = 1; s < ES; ++s)
+      if (n_ent > 64 * s && meta[s] >= 0 &&
+          (bm < 0 || key[s] > bk || (key[s] == bk && (r0[s] < b0 || (r0[s] == b0 && r1[s] < b1))))) {
+        bk = key[s];
+        b0 = r0[s];
+        b1 = r1[s];
+        bm = meta[s];
+        bs = s;
       }
+    bool in = bm >= 0;
+    unsigned long long win = __ballot(in);
+    if (win == 0ull) break;  // heap empty
+    auto narrow = [&](uint32_t v) {
+      const uint32_t m = wave_umax(in ? v : 0u);
+      in = in && v == m;
+      win = __ballot(in);
+    };
+    narrow((uint32_t)(bk >> 32));
+    if (win & (win - 1ull)) narrow((uint32_t)bk);
+    if (win & (win - 1ull)) {  // equal logw: the smaller rank tuple
+      narrow(~(uint32_t)(b0 >> 32));
+      narrow(~(uint32_t)b0);
+      narrow(~(uint32_t)(b1 >> 32));
+      narrow(~(uint32_t)b1);
+    }
+    const int src = __builtin_ctzll(win);
+    const double bl = key_logw(readlane64(bk, src));
+    const unsigned long long w0 = readlane64(b0, src), w1 = readlane64(b1, src);
+    const int m = __builtin_amdgcn_readlane(bm, src), slot = ES > 1 ? __builtin_amdgcn_readlane(bs, src) : 0;
+    const int parent = m & 255, d = (m >> 8) & 255, r = m >> 16, at = (d - 1) * p.k + r;
+    const int idx = ++nodes;
+    const int token = s_tok[at];
+    // Two new entries in two lanes' slots: the sibling with ranks[:-1] +
+    // (rank + 1,) and the first child with ranks + (0,).
+    const bool sib = r + 1 < p.k, child = d < p.depth;
+    const int es = n_ent, ec = n_ent + (sib ? 1 : 0);
+    n_ent = ec + (child ? 1 : 0);
+    const bool is_c = child && lane == (ec & 63);
+    const double lp_add = (double)s_lp[is_c ? d * p.k : at + (sib ? 1 : 0)];
+    const double base = is_c ? bl : bl - (double)s_lp[at];
+    const unsigned long long nk = ordered_key(base + lp_add);
+    unsigned long long q0 = w0, q1 = w1;
+    add_level(q0, q1, d + (is_c ? 1 : 0), 1ull);
+    const int nm = is_c ? idx | ((d + 1) << 8) : parent | (d << 8) | ((r + 1) << 16);
+    const int e = is_c ? ec : sib && lane == (es & 63) ? es : -1;
+#pragma unroll
+    for (int s = 0; s < ES; ++s) {
+      if (slot == s && lane == src) meta[s] = -1;
+      if (e >= 0 && (e >> 6) == s) {
+        key[s] = nk;
+        r0[s] = q0;
+        r1[s] = q1;
+        meta[s] = nm;
+      }
+    }
+    uint32_t a[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      a[w] = (uint32_t)__builtin_amdgcn_readlane((int)anc[0][w], parent & 63);
+#pragma unroll
+      for (int s = 1; s < NS; ++s)
+        if ((parent >> 6) == s) a[w] = (uint32_t)__builtin_amdgcn_readlane((int)anc[s][w], parent & 63);
+      if (w == idx / 32) a[w] |= 1u << (idx % 32);
     }
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const double ol = __shfl_xor(bl, o);
-      const unsigned long long o0 = __shfl_xor(b0, o), o1 = __shfl_xor(b1, o);
-      const int oi = __shfl_xor(bi, o);
-      if (oi >= 0 && (bi < 0 || better(ol, o0, o1, bl, b0, b1))) {
-        bl = ol;
-        b0 = o0;
-        b1 = o1;
-        bi = oi;
-      }
-    }
-    if (bi < 0) break;  // heap empty (every lane agrees)
-    const int meta = e_meta[bi];
-    const int parent = meta & 255, d = (meta >> 8) & 255, r = meta >> 16;
-    const int idx = nodes + 1;
-    if (lane == 0) {
-      e_meta[bi] = -1;
-      const int tok = p.top_tok[(d - 1) * p.k + r];
-      n_tok[idx] = tok;
-      n_par[idx] = parent;
-      n_dep[idx] = d;
+    for (int s = 0; s < NS; ++s)
+      if (lane + 64 * s == idx) {
+        tok[s] = token;
+        par[s] = parent;
+        dep[s] = d;
 #pragma unroll
-      for (int w = 0; w < DTREE_MASK_WORDS; ++w)
-        n_anc[idx][w] = (parent == 0 ? (w == 0 ? 1u : 0u) : n_anc[parent][w]) | (w == idx / 32 ? 1u << (idx % 32) : 0u);
-      int ne = n_ent;
-      if (r + 1 < p.k) {  // sibling: ranks[:-1] + (rank + 1,)
-        e_logw[ne] = (bl - (double)p.top_lp[(d - 1) * p.k + r]) + (double)p.top_lp[(d - 1) * p.k + r + 1];
-        unsigned long long s0 = b0, s1 = b1;
-        add_level(s0, s1, d, 1ull);
-        e_r0[ne] = s0;
-        e_r1[ne] = s1;
-        e_meta[ne] = parent | (d << 8) | ((r + 1) << 16);
-        ++ne;
+        for (int w = 0; w < NW; ++w) anc[s][w] = a[w];
       }
-      if (d < p.depth) {  // first child: ranks + (0,)
-        e_logw[ne] = bl + (double)p.top_lp[d * p.k];
-        unsigned long long c0 = b0, c1 = b1;
-        add_level(c0, c1, d + 1, 1ull);
-        e_r0[ne] = c0;
-        e_r1[ne] = c1;
-        e_meta[ne] = idx | ((d + 1) << 8);
-      }
-    }
-    n_ent += (r + 1 < p.k ? 1 : 0) + (d < p.depth ? 1 : 0);
-    ++nodes;
-    __syncthreads();
   }
   // descriptor: root + nodes in pop order, rows past L cleared
   const int L = nodes + 1;
   DtreeStepDesc* dd = p.desc;
-  for (int i = lane; i < DTREE_MAX_NODES; i += 64) {
-    const bool live = i < L;
-    dd->tokens[i] = !live ? 0 : (i == 0 ? p.root : n_tok[i]);
-    dd->positions[i] = !live ? 0 : p.past + (i == 0 ? 0 : n_dep[i]);
-    dd->parents[i] = !live ? -1 : (i == 0 ? -1 : n_par[i]);
 #pragma unroll
-    for (int w = 0; w < DTREE_MASK_WORDS; ++w)
-      dd->ancestors[i][w] = !live ? 0u : (i == 0 ? (w == 0 ? 1u : 0u) : n_anc[i][w]);
+  for (int s = 0; s < DTREE_MAX_NODES / 64; ++s) {
+    const int i = lane + 64 * s, sn = s < NS ? s : 0;
+    const bool has = s < NS;
+    dd->tokens[i] = has ? tok[sn] : 0;
+    dd->positions[i] = i < L ? p.past + dep[sn] : 0;
+    dd->parents[i] = has ? par[sn] : -1;
+#pragma unroll
+    for (int w = 0; w < DTREE_MASK_WORDS; ++w) dd->ancestors[i][w] = has && w < NW ? anc[sn][w < NW ? w : 0] : 0u;
     dd->accepted[i] = 0;
     dd->posterior[i] = 0;
-    if (p.tree_out && i < DTREE_MAX_NODES - 1) {
-      p.tree_out[1 + i] = i + 1 < L ? n_tok[i + 1] : 0;
-      p.tree_out[1 + DTREE_MAX_NODES + i] = i + 1 < L ? n_dep[i + 1] : 0;
-      p.tree_out[1 + 2 * DTREE_MAX_NODES + i] = i + 1 < L ? n_par[i + 1] : -1;
+    if (p.tree_out && i > 0) {
+      p.tree_out[i] = has ? tok[sn] : 0;
+      p.tree_out[DTREE_MAX_NODES + i] = has ? dep[sn] : 0;
+      p.tree_out[2 * DTREE_MAX_NODES + i] = has ? par[sn] : -1;
     }
   }
   if (lane == 0) {
@@ -479,7 +628,10 @@ extern "C" int dtree_tree_build(const float* logits, int32_t ld, int32_t depth, 
     topk_merge_kernel<<<depth, kThreads, 0, stream>>>(p);
     DTREE_LAUNCH_CHECK("tree_build: merge pass");
   }
-  heap_kernel<<<1, 64, 0, stream>>>(p);
+  // 1 + 2 budget heap entries and 1 + budget nodes, 64 to a slot
+  if (budget <= 31) heap_kernel<1, 1><<<1, 64, 0, stream>>>(p);
+  else if (budget <= 63) heap_kernel<2, 1><<<1, 64, 0, stream>>>(p);
+  else heap_kernel<4, 2><<<1, 64, 0, stream>>>(p);
   DTREE_LAUNCH_CHECK("tree_build: heap");
   return DTREE_OK;
 }
