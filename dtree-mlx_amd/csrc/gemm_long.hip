@@ -714,6 +714,8 @@ using Q128x256 = Tile<2, 2, 2, 4, 3>;
 using Q256x192 = Tile<2, 3, 4, 2, 3>;
 using Q256x256 = Tile<4, 2, 2, 4, 3>;
 using T128x128 = Tile<2, 2, 2, 2, 4>;      // bf16 weights
+using T64x64k = Tile<2, 1, 1, 2, 4, 2>;
+using T64x128k = Tile<2, 2, 1, 2, 4, 2>;
 using T128x128k = Tile<2, 2, 2, 2, 4, 2>;
 using T256x128 = Tile<2, 2, 4, 2, 6>;
 using T256x192 = Tile<2, 3, 4, 2, 5>;
@@ -731,12 +733,14 @@ using T256x384 = Tile<4, 3, 2, 4, 3>;
 // 48 / 42 / 53 / 61 / 70 / 85; N 12352 K 2560 102 / 89 / 112 / 77 / 81 / 103;
 // N 19456 K 2560 136 / 129 / 120 / 133 / 98 / 108; N 24576 K 4096 244 / 212 /
 // 201 / 209 / 243 / 186; 4096 rows, N 24576 K 4096: 950 / 827 / 775 / 699 /
-// 697 / 728. The two widest do not take the residual epilogue (its preloaded
+// 697 / 728. The two smallest are for short prompts (64x64 / 64x128 / 128x128):
+// 128 rows, N 6144 K 2560 14 / 17 / 21; 384 rows, N 2560 K 9728 38 / 48 / 56;
+// 768 rows, the same 65 / 54 / 60. The two widest do not take the residual epilogue (its preloaded
 // rows would not fit their registers).
 struct TileCost { int tm, tn; float cost; };
-enum { kT128x128, kT256x128, kT256x192, kT256x256, kT256x320, kT256x384, kTiles };
-constexpr TileCost kTileCost[kTiles] = {{128, 128, 0.55f}, {256, 128, 0.75f}, {256, 192, 1.08f},
-                                        {256, 256, 1.30f}, {256, 320, 1.62f}, {256, 384, 2.05f}};
+enum { kT64x64, kT64x128, kT128x128, kT256x128, kT256x192, kT256x256, kT256x320, kT256x384, kTiles };
+constexpr TileCost kTileCost[kTiles] = {{64, 64, 0.25f}, {64, 128, 0.35f}, {128, 128, 0.55f}, {256, 128, 0.75f},
+                                        {256, 192, 1.08f}, {256, 256, 1.30f}, {256, 320, 1.62f}, {256, 384, 2.05f}};
 // The same for q4 weights (one or two K blocks per stage; 128 x 128 tiles need
 // an even number of them). us at 1024 rows (128x128 / 128x256 / 256x192 /
 // 256x256): N 2560 K 9728 106 / 191 / 248 / 339; N 12352 K 2560 141 / 115 / 149
@@ -767,6 +771,8 @@ int launch_long_dense(LongParams p, int epi, bool h16, int cus, hipStream_t st) 
   if (!h16)
     return p.x_lo ? launch_tile<T128x128, kBf16Lo>(p, epi, st) : launch_tile<T128x128, kBf16>(p, epi, st);
   switch (pick_tile(kTileCost, 0, epi == DTREE_EPI_RESIDUAL ? kT256x320 : kTiles, p.rows, p.n, cus)) {
+    case kT64x64: return launch_tile<T64x64k, kF16>(p, epi, st);
+    case kT64x128: return launch_tile<T64x128k, kF16>(p, epi, st);
     case kT256x128: return launch_tile<T256x128, kF16>(p, epi, st);
     case kT256x192: return launch_tile<T256x192, kF16>(p, epi, st);
     case kT256x256: return launch_tile<T256x256, kF16>(p, epi, st);

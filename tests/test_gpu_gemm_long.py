@@ -1,6 +1,6 @@
 """dtree_gemm_long's tile shapes against a float64 product.
 
-The fp16 path picks one of six tile shapes by rows and columns; the cases
+The fp16 path picks one of eight tile shapes by rows and columns; the cases
 below reach every one of them, with ragged last row and column tiles, with
 fewer K stages than the pipeline holds, and with outputs too misaligned for
 the vector stores. Bounds: the fp32 accumulation of K products differs from
@@ -97,7 +97,14 @@ def test_long_tiles_match_float64(gpu_device, rows, n, epi, k):
     _long(gpu_device, rows, n, k, epi)
 
 
-@pytest.mark.parametrize("rows,n", [(128, 64), (1024, 12352), (640, 19520), (1024, 19520), (1152, 24640)])
+# short prompts: 64x64, 64x128 and 128x128 tiles, in one and two per CU
+@pytest.mark.parametrize("rows,n", [(128, 6144), (384, 2560), (256, 12288), (768, 2560), (896, 2432), (384, 6144)])
+@pytest.mark.parametrize("epi", [N.EPI_STORE_F32, N.EPI_RESIDUAL, N.EPI_SWIGLU, N.EPI_STORE_BF16])
+def test_long_small_tiles(gpu_device, rows, n, epi):
+    _long(gpu_device, rows, n, 192, epi)
+
+
+@pytest.mark.parametrize("rows,n", [(128, 64), (128, 12352), (1024, 12352), (640, 19520), (1024, 19520), (1152, 24640)])
 def test_long_tiles_64_column_tail(gpu_device, rows, n):
     _long(gpu_device, rows, n, 192, N.EPI_STORE_F32)
 
