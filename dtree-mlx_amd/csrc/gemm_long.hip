@@ -392,8 +392,12 @@ __global__ __launch_bounds__(T::THREADS) void long_kernel(LongParams p) {
 //
 // Measured against the kernel this one replaced (128 x 128 tiles through
 // registers, both folds as FMAs, sum(x) by MFMA in every wave): the 9B-shaped
-// MLP (gate/up and down) over 300 tokens 476 -> 248 us; N 24576, K 4096, 4096
-// rows 913 us (0.90 PFLOP/s; the fp16 tiles reach 1.18).
+// MLP (gate/up and down) over 300 tokens 477 -> 238 us; N 24576, K 4096, 4096
+// rows 846 us (0.98 PFLOP/s; the fp16 tiles reach 1.18). Bound by a wave's own
+// instruction chain (folds, unpacking, load issue, waits): a lone wave per SIMD
+// takes as long per stage as two, and deeper pipelines change nothing. With the
+// folds beginning under their block's last MFMA and the load resources remade
+// from vector registers at every load it was 248 us and 913 us.
 constexpr int kRing = 8;        // groups per correction step
 constexpr int kRingStride = 12; // floats per ring row (16-byte reads, spread over the banks)
 
@@ -480,14 +484,17 @@ __global__ __launch_bounds__(T::THREADS) void longq_kernel(LongParams p) {
     plds[j] = uni(lds0 + (pad ? NST * STAGE : 1024 * ch));
     pstage[j] = uni(pad ? 0u : ~0u);  // padding has one place for all stages
     pmask[j] = uni(isx || isw ? 0u : ~0u);  // scale words: eight lanes per column block
+    // opaque from here on: kept in scalar registers instead of being made again per stage
+    asm volatile("" : "+s"(plo[j]), "+s"(phi[j]), "+s"(psize[j]), "+s"(poff[j]), "+s"(pstep[j]), "+s"(plds[j]),
+                 "+s"(pstage[j]));
   }
   const unsigned lane16 = 16u * lane, lane_s = (unsigned)(lane >> 3) * nkb * 128u + 16u * (lane & 7) - lane16;
   // `at`: the stage's LDS offset. Past the last stage the size is 0 (no branch
   // and no select: the stage loop stays one block, as its order is written).
   auto issue = [&](int s, unsigned at, int j) {
     const uint32_t live = (uint32_t)((s - S) >> 31);
-    lds_load16(u32x4_t{plo[j], phi[j], psize[j] & live, 0x00020000u},
-               poff[j] + (unsigned)s * pstep[j] + lane16 + (lane_s & pmask[j]), plds[j] + (at & pstage[j]));
+    lds_load16_s(plo[j], phi[j], psize[j] & live, poff[j] + (unsigned)s * pstep[j] + lane16 + (lane_s & pmask[j]),
+                 plds[j] + (at & pstage[j]));
   };
   f32x16_t acc[NB][MB];
 #pragma unroll
@@ -536,9 +543,11 @@ __global__ __launch_bounds__(T::THREADS) void longq_kernel(LongParams p) {
 #pragma unroll
     for (int pl = 0; pl < NPL; ++pl) ssum[f & 1] = bf8_sum(sx[f * NPL + pl], f < 2 && pl == 0 ? 0.f : ssum[f & 1]);
   };
-  auto fold = [&](int v, int f, float scale) {  // a quarter of block v's sum
+  // A third of block v's sum, under the next block's MFMAs 1 .. 3 (its own last
+  // one is still running under MFMA 0).
+  auto fold = [&](int v, int f, float scale) {
 #pragma unroll
-    for (int r = 4 * f; r < 4 * f + 4; ++r)
+    for (int r = 16 * (f - 1) / 3; r < 16 * f / 3; ++r)
       acc[v % NB][v / NB][r] = fmaf(scale, au[v & 1][r], acc[v % NB][v / NB][r]);
   };
 #pragma unroll
@@ -602,8 +611,10 @@ __global__ __launch_bounds__(T::THREADS) void longq_kernel(LongParams p) {
             else read_a(nxt, 0, f, pl);
           }
         }
-        if (u > 0) fold(u - 1, f, sc[(u - 1) % NB]);
-        else fold(NT - 1, f, last);  // the previous stage's last block
+        if (f > 0) {
+          if (u > 0) fold(u - 1, f, sc[(u - 1) % NB]);
+          else fold(NT - 1, f, last);  // the previous stage's last block
+        }
         if (u + 1 < NB) unpack(u + 1, f);
         if (u + 1 == NT) unpack(0, f);
         if (u < 2 * NSUM) {
@@ -663,7 +674,7 @@ __global__ __launch_bounds__(T::THREADS) void longq_kernel(LongParams p) {
     }
   }
 #pragma unroll
-  for (int f = 0; f < 4; ++f) fold(NT - 1, f, sc[NB - 1]);
+  for (int f = 1; f < 4; ++f) fold(NT - 1, f, sc[NB - 1]);
   long_finish<T, EPI>(p, acc, smem, rs, wave, R, N0, [&](auto& a, float* buf) {
 #pragma unroll
     for (auto& aj : a)
@@ -743,11 +754,11 @@ constexpr TileCost kTileCost[kTiles] = {{64, 64, 0.25f}, {64, 128, 0.35f}, {128,
                                         {256, 192, 1.08f}, {256, 256, 1.30f}, {256, 320, 1.62f}, {256, 384, 2.05f}};
 // The same for q4 weights (one or two K blocks per stage; 128 x 128 tiles need
 // an even number of them). us at 1024 rows (128x128 / 128x256 / 256x192 /
-// 256x256): N 2560 K 9728 106 / 191 / 248 / 339; N 12352 K 2560 141 / 115 / 149
-// / 101; N 24576 K 4096 315 / 277 / 243 / 296; 4096 rows, N 24576 K 4096: 1211
-// / 1093 / 982 / 953.
+// 256x256): N 2560 K 9728 106 / 179 / 237 / 286; N 12352 K 2560 136 / 111 / 143
+// / 88; N 24576 K 4096 290 / 256 / 231 / 261; 4096 rows, N 24576 K 4096: 1141
+// / 1021 / 920 / 846; N 2560 K 9728: 316 / 369 / 259 / 289.
 enum { kQ128x128, kQ128x256, kQ256x192, kQ256x256, kQTiles };
-constexpr TileCost kQTileCost[kQTiles] = {{128, 128, 0.84f}, {128, 256, 1.42f}, {256, 192, 1.87f}, {256, 256, 2.40f}};
+constexpr TileCost kQTileCost[kQTiles] = {{128, 128, 0.75f}, {128, 256, 1.33f}, {256, 192, 1.80f}, {256, 256, 2.20f}};
 
 // The first of `count` shapes from `from` on with the least rounds x cost.
 int pick_tile(const TileCost* cost, int from, int count, int rows, int n, int cus) {

@@ -554,7 +554,8 @@ int dtree_gdn_layers_commit(const DtreeGdnArgs* args, int32_t num_layers, hipStr
  * forward_dflash, custom_qwen35_model.py:961-1097, through
  * Qwen35TargetAdapter.forward_with_hidden_states, adapters.py:290-307).
  * desc is unused; rows_padded is the row capacity of q, k, v, g, beta, y,
- * proj and out (num_tokens <= rows_padded). */
+ * proj and out (num_tokens <= rows_padded). out is also scratch between the
+ * launches. */
 int dtree_gdn_layer_chain(const DtreeGdnArgs* args, int32_t num_tokens, hipStream_t stream);
 
 /* Convert a row-major [n][k] bf16 matrix to DTREE_W_TILED (n % 32 == 0,
