@@ -1700,9 +1700,10 @@ __global__ __launch_bounds__(256) void gdn_chain_scan_kernel(GdnParams p, const 
 //
 // The 64 floats per (token, value head) of A and U rows live in the layer's
 // `out` buffer between the two launches (128 16-bit values per head and token;
-// the gated norm overwrites all of it after). Rows: A [32] then U [32]; the
-// upper right quarters, which are zero and never read as matrix, hold gamma
-// (of A: rows 0 and 1, tokens 0-15 and 16-31) and suf (of U).
+// the gated norm overwrites all of it after). Rows: A [32] then U [32]. The
+// upper right quarters, zero in both matrices, are not written: their first two
+// rows hold gamma (of A: tokens 0-15 and 16-31) and suf (of U), the others
+// what the buffer held before, and no product takes an operand from there.
 constexpr int kChainChunk = 32;
 struct ChainScratch {
   float* base;
@@ -1914,7 +1915,8 @@ __global__ __launch_bounds__(256, 1) void gdn_chain_chunk_kernel(GdnParams p, Ch
     o.a[1] = f4(&b.m[16 + n][4 * kk]);
     o.a[2] = f4(&b.m[16 + n][16 + 4 * kk]);
     o.u[0] = f4(&b.m[16 * ym + n][32 + 4 * kk]);
-    o.u[1] = f4(&b.m[16 * ym + n][48 + 4 * kk]);
+    // (U's upper right quarter is not in the scratch: zero, whatever lies there)
+    o.u[1] = ym ? f4(&b.m[16 + n][48 + 4 * kk]) : f32x4_t{0.f, 0.f, 0.f, 0.f};
   };
   // Chunk c from o. After its barrier every wave has read chunk c's stage and
   // chunk c + 1's is complete: the next operands come from there, and chunk

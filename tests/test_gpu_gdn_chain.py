@@ -2,8 +2,9 @@
 and beta (the prep is checked elsewhere): both forms around their boundary,
 ragged last chunks, long runs of one repeated token (equal keys, decays and
 betas near 1, where powers of the chunk matrix would grow like binomials),
-vanishing decays, head groups from 1 to 8, and row-major outputs without
-padding rows.
+vanishing decays, head groups from 1 to 8, row-major outputs without padding
+rows, and in every output layout an `out` buffer that holds NaN before the call
+(it is scratch between the launches, and its old contents must not matter).
 
 Bound: the recurrence is a contraction here (|k| = 1, beta and g in [0, 1]), so
 fp32 rounding of a few operations per token adds up to some 2^-24 sqrt(tokens)
@@ -18,7 +19,7 @@ from dtree_hip import _native as N
 pytestmark = pytest.mark.gpu
 
 
-def _chain(dev, T, Hk=16, Hv=32, kind="random", rowmajor=False):
+def _chain(dev, T, Hk=16, Hv=32, kind="random", rowmajor=False, h16=False, stale=False):
     g = torch.Generator(device=dev)
     g.manual_seed(T + Hk + 7 * Hv + len(kind))
     D = 128
@@ -42,7 +43,9 @@ def _chain(dev, T, Hk=16, Hv=32, kind="random", rowmajor=False):
     z = lambda *s, dtype=torch.float32: torch.zeros(*s, dtype=dtype, device=dev)  # noqa: E731
     b = dict(q=z(rows, key), k=z(rows, key), v=z(rows, val), g=z(rows, Hv), beta=z(rows, Hv), y=z(rows, val))
     ld = val + 8 if rowmajor else val
-    out = z(rows, ld, dtype=torch.bfloat16)
+    out = z(rows, ld, dtype=torch.float16 if h16 else torch.bfloat16)
+    if stale:  # NaN as 16-bit values and as the fp32 words of the scratch
+        out.view(torch.int16).fill_(-1)
     conv = torch.rand(4, Cd, device=dev, generator=g) - 0.5
     alog = torch.log(1.0 + 15.0 * torch.rand(Hv, device=dev, generator=g))
     norm = torch.ones(D, dtype=torch.bfloat16, device=dev)
@@ -55,8 +58,8 @@ def _chain(dev, T, Hk=16, Hv=32, kind="random", rowmajor=False):
     a.window, a.state, a.out = window.data_ptr(), state.data_ptr(), out.data_ptr()
     a.conv_w, a.A_log, a.dt_bias = conv.data_ptr(), alog.data_ptr(), dt_bias.data_ptr()
     a.norm_w, a.eps = norm.data_ptr(), 1e-6
-    a.out_layout, a.ld_out = (N.W_ROWMAJOR if rowmajor else N.W_TILED), ld
-    print(f"gdn chain T={T} Hk={Hk} Hv={Hv} {kind} rowmajor={rowmajor}", flush=True)
+    a.out_layout, a.ld_out = (N.W_ROWMAJOR if rowmajor else N.W_TILED_F16 if h16 else N.W_TILED), ld
+    print(f"gdn chain T={T} Hk={Hk} Hv={Hv} {kind} rowmajor={rowmajor} h16={h16} stale={stale}", flush=True)
     N.check(N.lib().dtree_gdn_layer_chain(C.byref(a), T, torch.cuda.current_stream().cuda_stream), "gdn chain")
     torch.cuda.synchronize()
     grp = Hv // Hk
@@ -85,7 +88,7 @@ def _chain(dev, T, Hk=16, Hv=32, kind="random", rowmajor=False):
         full = untile_weight(out).double()
         assert (full[T:] == 0).all()
         o = full[:T].reshape(T, Hv, D)
-    # bf16 rounding, and y's own error seen through its norm where y is small
+    # 16-bit rounding, and y's own error seen through its norm where y is small
     err = 2e-6 * y.norm() / y.norm(dim=-1, keepdim=True) * 8
     assert ((o - ref).abs() <= (2.0 ** -8 + err) * ref.abs() + 1e-5 + err).all()
 
@@ -109,3 +112,9 @@ def test_chain_head_groups(gpu_device, Hk, Hv):
 @pytest.mark.parametrize("T", [41, 64, 65, 81])
 def test_chain_row_major_unpadded(gpu_device, T):
     _chain(gpu_device, T, 2, 4, rowmajor=True)
+
+
+@pytest.mark.parametrize("layout", ["tiled", "tiled_f16", "rowmajor"])
+@pytest.mark.parametrize("T", [40, 41, 63, 65, 81, 300])
+def test_chain_ignores_old_out(gpu_device, T, layout):
+    _chain(gpu_device, T, 4, 8, rowmajor=layout == "rowmajor", h16=layout == "tiled_f16", stale=True)
