@@ -288,23 +288,49 @@ __global__ __launch_bounds__(T::THREADS) void long_kernel(LongParams p) {
   const unsigned strip = (unsigned)nkb * 4096u;  // bytes of one 32-row strip
   const size_t xo = (size_t)R * p.k, wo = (size_t)N0 * p.k;
   const unsigned xbytes = (unsigned)min(T::TM, p.rows - R) / 32u * strip;
+  const unsigned wbytes = (unsigned)min(T::TN, p.n - N0) / 32u * strip;
   const u32x4_t xr = strip_rsrc(p.x + xo, xbytes);
-  const u32x4_t xlr = strip_rsrc((NPL > 1 ? p.x_lo : p.x) + xo, xbytes);
-  const u32x4_t wr = strip_rsrc(p.w + wo, (unsigned)min(T::TN, p.n - N0) / 32u * strip);
+  const u32x4_t wr = strip_rsrc(p.w + wo, wbytes);
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
   // Piece wave + WAVES j of stage s: activation pieces (plane, row block,
   // fragment), then weight pieces (column block, fragment). Past the last
   // stage or piece the load reads nothing, so every wave always has the same
   // number in flight.
+  // Two planes: the piece's base, size, offset and place are kept in scalar
+  // registers. Chosen among three resources at every load they went through
+  // scratch, whose waits also wait for the stage loads just issued (N 19456,
+  // K 2560, 1024 rows: 1229 us, so 219). For one plane the choice between two
+  // is the faster form (N 2560, K 9728, 1024 rows, bf16: 79 us, in registers 82).
+  constexpr bool WORDS = NPL > 1;
+  uint32_t plo[PW], phi[PW], psize[PW], poff[PW];
+  if constexpr (WORDS) {
+    static_assert(!PAD, "two planes deal their pieces out evenly");
+#pragma unroll
+    for (int j = 0; j < PW; ++j) {
+      const int ch = wave + T::WAVES * j;
+      const bool isa = ch < ACH, low = isa && ch >= ACH / NPL;
+      const int ap = !isa ? ch - ACH : low ? ch - ACH / NPL : ch;
+      const uint64_t base = isa ? (uint64_t)((low ? p.x_lo : p.x) + xo) : (uint64_t)(p.w + wo);
+      plo[j] = uni((uint32_t)base);
+      phi[j] = uni((uint32_t)(base >> 32) & 0xffffu);
+      psize[j] = uni(isa ? xbytes : wbytes);
+      poff[j] = uni((unsigned)(ap / SUB) * strip + (unsigned)(ap % SUB) * 1024u);
+      // opaque from here on: kept instead of being made again per stage
+      asm volatile("" : "+s"(plo[j]), "+s"(phi[j]), "+s"(psize[j]), "+s"(poff[j]));
+    }
+  }
   auto issue = [&](int s, int j) {
     const int ch = wave + T::WAVES * j;
-    const bool isa = ch < ACH, pad = PAD && ch >= CH;
-    const int a = isa ? ch : ch - ACH;
-    const int plane = NPL > 1 && isa && a >= ACH / NPL;
-    const int ap = plane ? a - ACH / NPL : a;
-    const unsigned off = (unsigned)(ap / SUB) * strip + (unsigned)(ap % SUB + SUB * s) * 1024u;
-    const unsigned lds = lds0 + (pad ? (unsigned)(NST * STAGE) : (unsigned)((s % NST) * STAGE + 1024 * ch));
-    lds_load16(isa ? (plane ? xlr : xr) : wr, (s < S && !pad ? off : kOob) + 16u * lane, lds);
+    if constexpr (WORDS) {
+      lds_load16_s(plo[j], phi[j], psize[j] & (uint32_t)((s - S) >> 31),
+                   poff[j] + (unsigned)s * (SUB * 1024u) + 16u * lane, lds0 + (s % NST) * STAGE + 1024 * ch);
+    } else {
+      const bool isa = ch < ACH, pad = PAD && ch >= CH;
+      const int ap = isa ? ch : ch - ACH;
+      const unsigned off = (unsigned)(ap / SUB) * strip + (unsigned)(ap % SUB + SUB * s) * 1024u;
+      const unsigned lds = lds0 + (pad ? (unsigned)(NST * STAGE) : (unsigned)((s % NST) * STAGE + 1024 * ch));
+      lds_load16(isa ? xr : wr, (s < S && !pad ? off : kOob) + 16u * lane, lds);
+    }
   };
   f32x16_t acc[NB][MB];
 #pragma unroll

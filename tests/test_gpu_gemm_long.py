@@ -21,29 +21,42 @@ def _silu(t):
     return t * torch.sigmoid(t)
 
 
-def _long(dev, rows, n, k, epi, misaligned=False, seed=0):
+def _long(dev, rows, n, k, epi, misaligned=False, seed=0, form="f16"):
+    """form: fp16 operands, bf16 operands, or bf16 weights with the activations
+    and the outputs as split pairs of bf16 planes (value = hi + lo)."""
     g = torch.Generator(device=dev)
     g.manual_seed(seed + rows + 3 * n + 7 * k)
-    x = torch.empty(rows, k, device=dev).normal_(generator=g).half()
-    w = torch.empty(n, k, device=dev).normal_(0.0, 0.05, generator=g).half()
-    xt, wt = tile_weight_f16(x), tile_weight_f16(w)
+    h16, pair = form == "f16", form == "pair"
+    dt = torch.float16 if h16 else torch.bfloat16
+    x = torch.empty(rows, k, device=dev).normal_(generator=g)
+    xl = (x - x.to(dt).float()).to(dt)
+    x = x.to(dt)
+    w = torch.empty(n, k, device=dev).normal_(0.0, 0.05, generator=g).to(dt)
+    tile = tile_weight_f16 if h16 else tile_weight
+    xt, xlt, wt = tile(x), tile(xl), tile(w)
+    layout = N.W_TILED_F16 if h16 else N.W_TILED
     off = 1 if misaligned else 0  # rows of odd length from an odd element: no vector access is aligned
     width = n // 2 if epi == N.EPI_SWIGLU else n
     ld = width + off
     a = N.GemmArgs()
-    a.x = xt.data_ptr(); a.w = wt.data_ptr(); a.x_layout = a.w_layout = N.W_TILED_F16
+    a.x = xt.data_ptr(); a.w = wt.data_ptr(); a.x_layout = a.w_layout = layout
+    if pair:
+        a.x_lo = xlt.data_ptr()
+        x = x.double() + xl.double()
     a.ldx = k; a.rows_padded = rows; a.n = n; a.k = k; a.epilogue = epi
     a.norm_dim = k; a.eps = 1e-6
-    a.out_layout = N.W_ROWMAJOR if misaligned else N.W_TILED_F16
+    a.out_layout = N.W_ROWMAJOR if misaligned else layout
     f32 = torch.zeros(rows * (n + off) + off, device=dev).normal_(generator=g)
     res0 = f32[off:].view(rows, n + off)[:, :n].double().clone()
-    act = torch.zeros(rows * ld + off, dtype=torch.int16, device=dev)
+    act, actl = (torch.zeros(rows * ld + off, dtype=torch.int16, device=dev) for _ in range(2))
     hid = torch.zeros(rows * (n + off) + off, dtype=torch.bfloat16, device=dev)
     norm = (1 + 0.1 * torch.empty(n, device=dev).normal_(generator=g)).to(torch.bfloat16)
     ss = torch.rand(rows // 32, k // 32, 32, device=dev, generator=g) + 0.5
     sso = torch.zeros(rows // 32, n // 32, 32, device=dev)
     a.out_f32 = f32.data_ptr() + 4 * off; a.ld_out_f32 = n + off
     a.out_bf16 = act.data_ptr() + 2 * off; a.ld_out_bf16 = ld
+    if pair:
+        a.out_lo = actl.data_ptr() + 2 * off
     rs = torch.ones(rows, dtype=torch.float64, device=dev)
     if epi == N.EPI_RESIDUAL:
         a.next_norm = norm.data_ptr(); a.ss_out = sso.data_ptr()
@@ -51,18 +64,18 @@ def _long(dev, rows, n, k, epi, misaligned=False, seed=0):
     else:
         a.ss_in = ss.data_ptr(); a.ss_tiles = k // 32
         rs = torch.rsqrt(ss.double().transpose(1, 2).reshape(rows, -1).sum(1) / k + 1e-6)
-    print(f"gemm_long rows={rows} n={n} k={k} epi={epi} misaligned={misaligned}", flush=True)
+    print(f"gemm_long rows={rows} n={n} k={k} epi={epi} misaligned={misaligned} {form}", flush=True)
     N.check(N.lib().dtree_gemm_long(C.byref(a), torch.cuda.current_stream().cuda_stream), "gemm_long")
     torch.cuda.synchronize()
     acc = x.double() @ w.double().T
     bound = (x.double().abs() @ w.double().abs().T).max().item() * k * 2.0 ** -24 * rs.max().item() + 1e-6
     f = f32[off:].view(rows, n + off)[:, :n].double()
     if misaligned:  # row-major bf16
-        b = act[off:].view(rows, ld)[:, :width].view(torch.bfloat16).double()
-        rnd = 2.0 ** -8
+        b = sum(t[off:].view(rows, ld)[:, :width].view(torch.bfloat16).double() for t in (act, actl))
     else:
-        b = untile_weight(act.view(torch.float16).view(rows, width)).double()
-        rnd = 2.0 ** -11
+        b = sum(untile_weight(t.view(dt).view(rows, width)).double() for t in (act, actl))
+    # (each plane of a pair rounds what it is given by 2^-8 at most)
+    rnd = 2.0 ** -16 if pair else 2.0 ** -11 if h16 and not misaligned else 2.0 ** -8
     if epi == N.EPI_STORE_F32:
         assert (f - acc * rs[:, None]).abs().max().item() <= bound
     elif epi == N.EPI_STORE_BF16:
@@ -95,6 +108,21 @@ SHAPES = [(128, 256), (1152, 6144), (640, 19456), (1152, 12416), (1024, 19456), 
 @pytest.mark.parametrize("k", [64, 320])
 def test_long_tiles_match_float64(gpu_device, rows, n, epi, k):
     _long(gpu_device, rows, n, k, epi)
+
+
+# bf16 weights, with one and two activation planes: 128x128 tiles, several per
+# CU and a K loop shorter and longer than the pipeline
+@pytest.mark.parametrize("form", ["bf16", "pair"])
+@pytest.mark.parametrize("rows,n,k", [(128, 256, 64), (384, 384, 128), (640, 512, 320), (1152, 6144, 192)])
+@pytest.mark.parametrize("epi", [N.EPI_STORE_F32, N.EPI_RESIDUAL, N.EPI_SWIGLU, N.EPI_STORE_BF16])
+@pytest.mark.parametrize("misaligned", [False, True])
+def test_long_bf16_matches_float64(gpu_device, rows, n, k, epi, form, misaligned):
+    _long(gpu_device, rows, n, k, epi, misaligned=misaligned, form=form)
+
+
+@pytest.mark.parametrize("form", ["bf16", "pair"])
+def test_long_bf16_64_column_tail(gpu_device, form):
+    _long(gpu_device, 256, 448, 192, N.EPI_STORE_F32, form=form)
 
 
 # short prompts: 64x64, 64x128 and 128x128 tiles, in one and two per CU
