@@ -14,6 +14,9 @@
 //   and P goes to the second product straight from the registers of the first.
 //   q and P are split pairs of bf16 (16 significant bits); K and V are the
 //   cache's bf16 values.
+// * Few rows over a long prefix are split over key ranges (causal_parts): a
+//   workgroup walks one range of its rows' pages and leaves O, m and l in fp32
+//   in the caller's workspace, and causal_combine_kernel adds the ranges.
 // * Row blocks with the longest ranges start first; the groups alternate, so a
 //   group's workgroups share an XCD's L2 when the groups divide the eight.
 //
@@ -22,7 +25,13 @@
 // of 32 clocks. Measured, 32 heads of 128, 8 groups, 1000 rows, no prefix: 48 us
 // + 6 us append, where a tree-attention launch per 128 rows took 194 us in eight
 // launches; 16 gated heads of 256, 4 groups, 4096 rows: 369 us in one segment,
-// 0.96 ms in four of 1024, where the launches per 128 rows took 1.95 ms.
+// 0.96 ms in four of 1024, where the launches per 128 rows took 1.95 ms. Key
+// ranges, 8192-key prefix, without / with them: 32 heads of 128, 128 rows 281 /
+// 64 us, 512 rows 293 / 170; 16 gated heads of 256, 128 rows 591 / 78 us, 512
+// rows 610 / 186, 1000 rows 659 / 350 (a tree-attention launch per 128 rows: 70,
+// 272; 83, 325, 673).
+#include <algorithm>
+
 #include "lds_load.h"
 
 namespace dtree {
@@ -38,7 +47,49 @@ struct CausalParams {
   uint16_t* out; uint16_t* out_lo; int ld_out, out_tiled, out_h16;
   int Hq, Hkv, past, n, rows;  // rows: n padded to whole 32-row blocks
   float scale_log2;
+  int parts;  // key ranges per workgroup of rows (1: the kernel writes `out` itself)
+  float* part; float* part_ml;  // of every (range, workgroup, wave): O^T fragments [32 D], m and l [2][32]
 };
+
+// Workgroup w of a group takes (row block, head) pairs 4 w .. 4 w + 3, a wave
+// each; `items` pairs per group.
+__host__ __device__ __forceinline__ int causal_groups(int items) { return (items + 3) / 4; }
+
+// Pages that workgroup w's rows need.
+__device__ __forceinline__ int causal_tiles(const CausalParams& p, int w, int G, int items) {
+  const int rbl = min(4 * w + 3, items - 1) / G;  // the workgroup's last row block
+  return (min(p.past + 32 * (rbl + 1), p.past + p.n) + DTREE_PAGE - 1) / DTREE_PAGE;
+}
+
+// Pages of one of its key ranges (the last may be shorter, ranges past it empty).
+constexpr int kMinRange = 2;
+__host__ __device__ __forceinline__ int causal_range(int tiles, int parts) {
+  const int per = (tiles + parts - 1) / parts;
+  return per > kMinRange ? per : kMinRange;
+}
+
+// A lane's values of dims 32 db .. of its row: scaled, gated, stored.
+template <int D, bool GATED>
+__device__ __forceinline__ void causal_store(const CausalParams& p, const f32x16_t& o, float inv, int row, int hq, int db,
+                                             int h) {
+  const bool valid = row < p.n;
+  const float* gate = p.qkv + (size_t)row * p.ld_qkv + hq * p.q_stride + D;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int d = 32 * db + 8 * q + 4 * h;
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = valid ? o[4 * q + e] * inv : 0.f;
+    if constexpr (GATED) {
+      const f32x4_t gt = *reinterpret_cast<const f32x4_t*>(gate + d);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = valid ? y[e] / (1.0f + __expf(-gt[e])) : 0.f;
+    }
+    const int col = hq * D + d;
+    const size_t oi = p.out_tiled ? tiled_index(row, col, p.ld_out) : (size_t)row * p.ld_out + col;
+    store_act4(p.out, p.out_lo, oi, y, p.out_h16);
+  }
+}
 
 // K / V rows of the segment into the cache. A workgroup owns one page of one KV
 // head: four threads per K row (RMSNorm, RoPE pairs inside a thread, 16-byte
@@ -136,15 +187,17 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void causal_attn_kernel(Caus
   __shared__ __attribute__((aligned(1024))) unsigned char smem[2][2 * PB];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int G = p.Hq / p.Hkv, items = G * (p.rows / 32), nw = (items + 3) / 4;
-  const int g = blockIdx.x % p.Hkv, w = nw - 1 - blockIdx.x / p.Hkv;
+  // key ranges cover the live rows alone (causal_combine_kernel writes all rows)
+  const int G = p.Hq / p.Hkv, items = G * ((p.parts > 1 ? p.n + 31 : p.rows) / 32), nw = causal_groups(items);
+  const int g = blockIdx.x % p.Hkv, b = blockIdx.x / p.Hkv, w = nw - 1 - b / p.parts, part = b % p.parts;
   const int item = 4 * w + wave, rb = item / G, hq = g * G + item % G;
   const int row0 = 32 * rb, row = row0 + c;
   const bool live = item < items && row0 < p.n;
   const int end = p.past + p.n;                                         // keys in the cache
   const int kend = live ? min(p.past + row0 + 32, end) : 0;             // keys this wave needs
-  const int rbl = min(4 * w + 3, items - 1) / G;                        // the workgroup's last row block
-  const int tiles = (min(p.past + 32 * (rbl + 1), end) + DTREE_PAGE - 1) / DTREE_PAGE;
+  const int all = causal_tiles(p, w, G, items), per = causal_range(all, p.parts);
+  const int first = part * per, tiles = p.parts > 1 ? min(all, first + per) : all;
+  if (p.parts > 1 && first >= tiles) return;  // (uniform; the ranges are counted alike in the combine)
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&smem[0][0];
   auto issue = [&](int t) {
     const size_t blk = ((size_t)p.page_table[t] * p.Hkv + g) * (DTREE_PAGE * D);
@@ -155,7 +208,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void causal_attn_kernel(Caus
 #pragma unroll
     for (int i = 0; i < PW / 2; ++i) lds_load16(vr, wave * (PW * 512) + 1024 * i + 16 * lane, lds + PB + 1024 * i);
   };
-  issue(0);
+  issue(first);
   // This lane's dims 16 j + 8 h .. + 7 of its query row: q_norm, RoPE (pairs j,
   // j + R / 32 in one lane), softmax scale in log2 units, split.
   u32x4_t qh[NJ], ql[NJ];
@@ -212,7 +265,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void causal_attn_kernel(Caus
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
   float m_run = kNegInf, l_run = 0.f;
-  for (int t = 0; t < tiles; ++t) {
+  for (int t = first; t < tiles; ++t) {
     stage_wait<0>();  // page t has landed for every wave, and every wave has read page t - 1
     if (t + 1 < tiles) issue(t + 1);
     const int k0 = DTREE_PAGE * t;
@@ -278,26 +331,61 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void causal_attn_kernel(Caus
   }
   if (item >= items) return;
   const float l = l_run + __shfl_xor(l_run, 32);
-  const bool valid = row < p.n;
-  const float inv = valid ? 1.f / l : 0.f;
-  const float* gate = p.qkv + (size_t)row * p.ld_qkv + hq * p.q_stride + D;
+  if (p.parts > 1) {
+    const size_t u = ((size_t)(part * nw + w) * p.Hkv + g) * 4 + wave;
+    f32x4_t* po = reinterpret_cast<f32x4_t*>(p.part + u * (32 * D)) + lane;
 #pragma unroll
-  for (int db = 0; db < ND; ++db)
+    for (int db = 0; db < ND; ++db)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int d = 32 * db + 8 * q + 4 * h;
-      float y[4];
+      for (int q = 0; q < 4; ++q)
+        po[(4 * db + q) * 64] = f32x4_t{o[db][4 * q], o[db][4 * q + 1], o[db][4 * q + 2], o[db][4 * q + 3]};
+    p.part_ml[u * 64 + lane] = h ? l : m_run;
+    return;
+  }
+  const float inv = row < p.n ? 1.f / l : 0.f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) y[e] = valid ? o[db][4 * q + e] * inv : 0.f;
-      if constexpr (GATED) {
-        const f32x4_t gt = *reinterpret_cast<const f32x4_t*>(gate + d);
+  for (int db = 0; db < ND; ++db) causal_store<D, GATED>(p, o[db], inv, row, hq, db, h);
+}
+
+// The key ranges' partial results into `out`: a wave per 32 dims of a (row
+// block, head) pair, the lanes as in the kernel above, so every partial is read
+// as whole kilobytes. A range whose keys lie past a row contributes nothing to
+// it (its weight is 0 next to the first range's, which holds key 0).
+template <int D, bool GATED>
+__global__ __launch_bounds__(256) void causal_combine_kernel(CausalParams p) {
+  constexpr int ND = D / 32;
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);  // (row block, head, dims), dims fastest
+  const int db = unit % ND, hq = unit / ND % p.Hq, rb = unit / ND / p.Hq;
+  if (32 * rb >= p.rows) return;
+  const int G = p.Hq / p.Hkv, g = hq / G, item = rb * G + hq % G, items = G * ((p.n + 31) / 32);
+  const int nw = causal_groups(items), w = item / 4, row = 32 * rb + c;
+  f32x16_t o;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = valid ? y[e] / (1.0f + __expf(-gt[e])) : 0.f;
+  for (int r = 0; r < 16; ++r) o[r] = 0.f;
+  float inv = 0.f;
+  if (32 * rb < p.n) {
+    const int all = causal_tiles(p, w, G, items), per = causal_range(all, p.parts), used = (all + per - 1) / per;
+    const size_t u0 = ((size_t)w * p.Hkv + g) * 4 + item % 4, du = (size_t)nw * p.Hkv * 4;
+    const float* ml = p.part_ml + u0 * 64 + c;
+    float m = kNegInf, l = 0.f;
+#pragma unroll 4
+    for (int s = 0; s < used; ++s) m = fmaxf(m, ml[s * du * 64]);
+    const f32x4_t* po = reinterpret_cast<const f32x4_t*>(p.part + u0 * (32 * D)) + 256 * db + lane;
+#pragma unroll 4
+    for (int s = 0; s < used; ++s) {
+      const float k = fast_exp2(ml[s * du * 64] - m);
+      l += k * ml[s * du * 64 + 32];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4_t v = po[s * du * (8 * D) + 64 * q];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[4 * q + e] = fmaf(k, v[e], o[4 * q + e]);
       }
-      const int col = hq * D + d;
-      const size_t oi = p.out_tiled ? tiled_index(row, col, p.ld_out) : (size_t)row * p.ld_out + col;
-      store_act4(p.out, p.out_lo, oi, y, p.out_h16);
     }
+    inv = row < p.n ? 1.f / l : 0.f;
+  }
+  causal_store<D, GATED>(p, o, inv, row, hq, db, h);
 }
 
 __global__ __launch_bounds__(256) void rope_positions_kernel(int first, int rows, int half, float base, float* cos_out,
@@ -309,6 +397,21 @@ __global__ __launch_bounds__(256) void rope_positions_kernel(int first, int rows
   const double ang = (double)(first + m) * inv;
   cos_out[e] = (float)cos(ang);
   sin_out[e] = (float)sin(ang);
+}
+
+// Workgroups that fill an MI355X's 256 CUs once. A workgroup walks its pages one
+// after another and uses its CU's matrix cores by itself (head_dim 128, 2048 rows
+// over 8192 keys: two on every CU, 4.2 us a page; 300 rows, one on a third of
+// them: 2.1), so rows that leave CUs idle are split over key ranges up to this
+// many workgroups.
+constexpr int kFill = 256;
+
+// Workspace of one key range of every workgroup.
+size_t causal_part_bytes(int D, int groups) { return (size_t)groups * 4 * (32 * D + 64) * sizeof(float); }
+
+int causal_parts(int groups, int past, int n) {
+  const int pages = (past + n + DTREE_PAGE - 1) / DTREE_PAGE;
+  return std::max(1, std::min(kFill / groups, pages / kMinRange));
 }
 
 }  // namespace
@@ -328,8 +431,12 @@ extern "C" int dtree_rope_positions(int32_t first_position, int32_t rows, int32_
   return DTREE_OK;
 }
 
-extern "C" int dtree_causal_attention(const DtreeAttnArgs* a, int32_t past_length, int32_t num_rows,
-                                      hipStream_t stream) {
+extern "C" size_t dtree_causal_attention_workspace_bytes(int32_t head_dim) {
+  return head_dim > 0 ? causal_part_bytes(head_dim, kFill) : 0;
+}
+
+extern "C" int dtree_causal_attention_split(const DtreeAttnArgs* a, int32_t past_length, int32_t num_rows,
+                                            void* workspace, size_t workspace_bytes, hipStream_t stream) {
   DTREE_REQUIRE(a, "causal_attention: null args");
   DTREE_REQUIRE(a->qkv && a->rope_cos && a->rope_sin && a->k_pages && a->v_pages && a->page_table && a->out,
                 "causal_attention: null pointer");
@@ -366,19 +473,33 @@ extern "C" int dtree_causal_attention(const DtreeAttnArgs* a, int32_t past_lengt
   p.out_tiled = a->out_layout != DTREE_W_ROWMAJOR;
   p.Hq = a->num_heads; p.Hkv = a->num_kv_heads; p.past = past_length; p.n = num_rows; p.rows = a->rows_padded;
   p.scale_log2 = a->scale * 1.4426950408889634f;
+  const int live = causal_groups(G * ((num_rows + 31) / 32)) * p.Hkv;
+  p.parts = causal_parts(live, past_length, num_rows);
+  // without room for two ranges, one: the kernel then needs no workspace
+  const size_t fit = workspace && ((uintptr_t)workspace & 15) == 0 ? workspace_bytes / causal_part_bytes(D, live) : 0;
+  if ((size_t)p.parts > fit) p.parts = std::max(1, (int)fit);
+  p.part = static_cast<float*>(workspace);
+  if (p.part) p.part_ml = p.part + (size_t)p.parts * live * 4 * (32 * D);
   const int pages = (past_length + num_rows - 1) / DTREE_PAGE - past_length / DTREE_PAGE + 1;
-  const long long groups = ((long long)(p.Hq / p.Hkv) * (p.rows / 32) + 3) / 4;
   const dim3 agrid(pages, p.Hkv);
-  const int grid = (int)(groups * p.Hkv);
+  const int grid = p.parts > 1 ? live * p.parts : causal_groups(G * (p.rows / 32)) * p.Hkv;
+  const int cgrid = (p.rows / 32 * p.Hq * (D / 32) + 3) / 4;
   if (D == 128) {
     causal_append_kernel<128, 128><<<agrid, 256, 0, stream>>>(p);
     DTREE_LAUNCH_CHECK("causal_attention append launch");
     causal_attn_kernel<128, 128, false><<<grid, 256, 0, stream>>>(p);
+    if (p.parts > 1) causal_combine_kernel<128, false><<<cgrid, 256, 0, stream>>>(p);
   } else {
     causal_append_kernel<256, 64><<<agrid, 256, 0, stream>>>(p);
     DTREE_LAUNCH_CHECK("causal_attention append launch");
     causal_attn_kernel<256, 64, true><<<grid, 256, 0, stream>>>(p);
+    if (p.parts > 1) causal_combine_kernel<256, true><<<cgrid, 256, 0, stream>>>(p);
   }
   DTREE_LAUNCH_CHECK("causal_attention launch");
   return DTREE_OK;
+}
+
+extern "C" int dtree_causal_attention(const DtreeAttnArgs* a, int32_t past_length, int32_t num_rows,
+                                      hipStream_t stream) {
+  return dtree_causal_attention_split(a, past_length, num_rows, nullptr, 0, stream);
 }

@@ -130,6 +130,8 @@ SIGNATURES = {
     "dtree_tree_attention": (C.c_int, [C.POINTER(AttnArgs), _vp]),
     "dtree_tree_attention_noalloc_max_bytes": (_sz, []),
     "dtree_tree_attention_noalloc": (C.c_int, [C.POINTER(AttnArgs), _vp]),
+    "dtree_causal_attention_split": (C.c_int, [C.POINTER(AttnArgs), _i32, _i32, _vp, _sz, _vp]),
+    "dtree_causal_attention_workspace_bytes": (_sz, [_i32]),
     "dtree_causal_attention": (C.c_int, [C.POINTER(AttnArgs), _i32, _i32, _vp]),
     "dtree_rope_positions": (C.c_int, [_i32, _i32, _i32, _f32, _vp, _vp, _vp]),
     "dtree_attention_status": (C.c_int, [_vp, _vp, _vp]),

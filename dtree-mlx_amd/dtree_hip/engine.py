@@ -338,7 +338,9 @@ class TreeEngineBase:
         a.rows_padded = rows; a.scale = c.head_dim ** -0.5
         for name, v in geometry.items():
             setattr(a, name, v)
-        N.check(self.lib.dtree_causal_attention(C.byref(a), P0, n, st), "prefill attention")
+        ws = pf["attn_ws"]
+        N.check(self.lib.dtree_causal_attention_split(C.byref(a), P0, n, ws.data_ptr(), ws.numel(), st),
+                "prefill attention")
 
     def _prefill_logits(self, pf: dict, n: int, st: int) -> torch.Tensor:
         """fp32 logits [1, 1, V] of a segment's last row (its xg / ss rows hold
@@ -722,7 +724,9 @@ class Qwen3TreeEngine(TreeEngineBase):
                   act=torch.zeros(2, rows, F, dtype=self.act_dtype, device=dev),
                   hidden=torch.zeros(rows, nh * H, dtype=bf16, device=dev),
                   cos=torch.zeros(rows, D // 2, dtype=f32, device=dev),
-                  sin=torch.zeros(rows, D // 2, dtype=f32, device=dev))
+                  sin=torch.zeros(rows, D // 2, dtype=f32, device=dev),
+                  attn_ws=torch.empty(self.lib.dtree_causal_attention_workspace_bytes(c.head_dim), dtype=torch.uint8,
+                                      device=dev))
         self._pf = pf
         return pf
 

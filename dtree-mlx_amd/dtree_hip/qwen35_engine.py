@@ -265,7 +265,9 @@ class Qwen35TreeEngine(TreeEngineBase):
                   act=torch.zeros(2, rows, F, dtype=self.act_dtype, device=dev),
                   hidden=torch.zeros(rows, nh * H, dtype=bf16, device=dev),
                   cos=torch.zeros(rows, c.rope_dims // 2, dtype=f32, device=dev),
-                  sin=torch.zeros(rows, c.rope_dims // 2, dtype=f32, device=dev))
+                  sin=torch.zeros(rows, c.rope_dims // 2, dtype=f32, device=dev),
+                  attn_ws=torch.empty(self.lib.dtree_causal_attention_workspace_bytes(c.head_dim), dtype=torch.uint8,
+                                      device=dev))
         self._pf = pf
         return pf
 

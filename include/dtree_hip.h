@@ -375,6 +375,13 @@ int dtree_embed_tokens(const int32_t* tokens, int32_t n, const uint16_t* embed, 
  * dtree_rope_table does for a tree's positions.
  */
 int dtree_causal_attention(const DtreeAttnArgs* args, int32_t past_length, int32_t num_rows, hipStream_t stream);
+/* The same, with few rows over a long prefix split over key ranges. Their
+ * partial results lie in `workspace` (16-byte aligned, any contents, up to
+ * dtree_causal_attention_workspace_bytes; a buffer of its own, not the tree
+ * attention's). With less room fewer ranges are used, down to one. */
+size_t dtree_causal_attention_workspace_bytes(int32_t head_dim);
+int dtree_causal_attention_split(const DtreeAttnArgs* args, int32_t past_length, int32_t num_rows, void* workspace,
+                                 size_t workspace_bytes, hipStream_t stream);
 int dtree_rope_positions(int32_t first_position, int32_t rows, int32_t rope_dims, float rope_base, float* rope_cos,
                          float* rope_sin, hipStream_t stream);
 

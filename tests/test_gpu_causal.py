@@ -28,12 +28,15 @@ def _rope(x, pos, dims, base):
     return torch.cat([a * c - b * s, a * s + b * c, x[..., dims:]], -1)
 
 
-def _case(dev, geo, Hq, Hkv, past, n, tiled=True, norms=True):
+def _case(dev, geo, Hq, Hkv, past, n, tiled=True, norms=True, workspace=None, pad=32):
+    """workspace: None, or (bytes, misalignment) for dtree_causal_attention_split;
+    returns the share of the workspace that the call wrote. pad: rows of qkv and
+    out come in multiples of it."""
     D, R, gated = (128, 128, 0) if geo == "qwen3" else (256, 64, 1)
     g = torch.Generator(device=dev)
     g.manual_seed(past * 1000 + n + Hq)
     rnd = lambda *s: torch.empty(*s, device=dev).normal_(generator=g)  # noqa: E731
-    rows = 32 * ((n + 31) // 32)
+    rows = pad * ((n + pad - 1) // pad)
     qs = D * (2 if gated else 1)
     ld = Hq * qs + 2 * Hkv * D
     qkv = torch.zeros(rows, ld, device=dev)
@@ -64,8 +67,13 @@ def _case(dev, geo, Hq, Hkv, past, n, tiled=True, norms=True):
     a.ld_out = width; a.out_layout = N.W_TILED if tiled else N.W_ROWMAJOR
     a.num_heads, a.num_kv_heads, a.head_dim, a.rows_padded = Hq, Hkv, D, rows
     a.scale = D ** -0.5; a.rope_dims = R; a.gated = gated
-    print(f"causal attention {geo} Hq={Hq} Hkv={Hkv} past={past} n={n} tiled={tiled}", flush=True)
-    N.check(N.lib().dtree_causal_attention(C.byref(a), past, n, st), "causal attention")
+    print(f"causal attention {geo} Hq={Hq} Hkv={Hkv} past={past} n={n} tiled={tiled} {workspace}", flush=True)
+    if workspace is None:
+        N.check(N.lib().dtree_causal_attention(C.byref(a), past, n, st), "causal attention")
+    else:
+        ws = torch.full((workspace[0] // 4 + 4,), float("nan"), device=dev)
+        N.check(N.lib().dtree_causal_attention_split(C.byref(a), past, n, ws.data_ptr() + workspace[1], workspace[0],
+                                                     st), "causal attention")
     torch.cuda.synchronize()
 
     x = qkv[:n].double()
@@ -97,6 +105,42 @@ def _case(dev, geo, Hq, Hkv, past, n, tiled=True, norms=True):
     assert (o[n:] == 0).all()
     err = ((o[:n] - ref.reshape(n, -1)).norm() / ref.norm()).item()
     assert err <= 2e-4, err
+    if workspace is not None:
+        assert torch.isnan(ws[workspace[0] // 4:]).all()
+        return 1 - torch.isnan(ws).double().mean().item()
+
+
+# partial results of one key range: per workgroup (four 32-row units), O and two statistics
+def _range_bytes(Hq, Hkv, D, n):
+    return Hkv * ((Hq // Hkv * ((n + 31) // 32) + 3) // 4) * 4 * (32 * D + 64) * 4
+
+
+@pytest.mark.parametrize("geo,D", [("qwen3", 128), ("gated", 256)])
+@pytest.mark.parametrize("past,n", [(300, 1), (0, 200), (1000, 31), (4095, 33), (1985, 130), (127, 513)])
+def test_causal_key_ranges(gpu_device, geo, D, past, n):
+    """Prefixes that end inside a page, rows whose first keys lie past some
+    ranges, empty last ranges; pages the segment does not own hold NaN."""
+    full = N.lib().dtree_causal_attention_workspace_bytes(D)
+    assert _case(gpu_device, geo, 8, 2, past, n, workspace=(full, 0)) > 0
+
+
+@pytest.mark.parametrize("geo,D,Hq,Hkv", [("qwen3", 128, 12, 3), ("qwen3", 128, 16, 2), ("gated", 256, 10, 5)])
+def test_causal_key_ranges_groups(gpu_device, geo, D, Hq, Hkv):
+    full = N.lib().dtree_causal_attention_workspace_bytes(D)
+    assert _case(gpu_device, geo, Hq, Hkv, 700, 70, tiled=False, workspace=(full, 0), pad=128) > 0
+
+
+@pytest.mark.parametrize("geo,D", [("qwen3", 128), ("gated", 256)])
+@pytest.mark.parametrize("ranges,used", [(3, True), (2, True), (1, False), (0, False)])
+def test_causal_short_workspace(gpu_device, geo, D, ranges, used):
+    """No more ranges than the workspace holds; less than two: none."""
+    size = ranges * _range_bytes(8, 2, D, 40)
+    assert (_case(gpu_device, geo, 8, 2, 900, 40, workspace=(size, 0)) > 0) == used
+
+
+def test_causal_misaligned_workspace_is_not_used(gpu_device):
+    full = N.lib().dtree_causal_attention_workspace_bytes(128)
+    assert _case(gpu_device, "qwen3", 8, 2, 900, 40, workspace=(full, 4)) == 0
 
 
 @pytest.mark.parametrize("geo", ["qwen3", "gated"])
