@@ -180,7 +180,8 @@ __device__ __forceinline__ u32x4_t clip_keys(u32x4_t v, int first, int end) {
   return v;
 }
 
-template <int D, int R, bool GATED>
+// SPLIT: one of p.parts key ranges of the rows, to the workspace.
+template <int D, int R, bool GATED, bool SPLIT>
 __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void causal_attn_kernel(CausalParams p) {
   constexpr int NJ = D / 16, ND = D / 32, PB = DTREE_PAGE * D * 2;  // bytes of a page's K (or V)
   constexpr int PW = 2 * PB / 1024 / 4;                             // 1 KB pieces per wave and page
@@ -188,16 +189,21 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void causal_attn_kernel(Caus
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // key ranges cover the live rows alone (causal_combine_kernel writes all rows)
-  const int G = p.Hq / p.Hkv, items = G * ((p.parts > 1 ? p.n + 31 : p.rows) / 32), nw = causal_groups(items);
-  const int g = blockIdx.x % p.Hkv, b = blockIdx.x / p.Hkv, w = nw - 1 - b / p.parts, part = b % p.parts;
+  const int G = p.Hq / p.Hkv, items = G * ((SPLIT ? p.n + 31 : p.rows) / 32), nw = causal_groups(items);
+  const int g = blockIdx.x % p.Hkv, b = blockIdx.x / p.Hkv, part = SPLIT ? b % p.parts : 0;
+  const int w = nw - 1 - (SPLIT ? b / p.parts : b);
   const int item = 4 * w + wave, rb = item / G, hq = g * G + item % G;
   const int row0 = 32 * rb, row = row0 + c;
   const bool live = item < items && row0 < p.n;
   const int end = p.past + p.n;                                         // keys in the cache
   const int kend = live ? min(p.past + row0 + 32, end) : 0;             // keys this wave needs
-  const int all = causal_tiles(p, w, G, items), per = causal_range(all, p.parts);
-  const int first = part * per, tiles = p.parts > 1 ? min(all, first + per) : all;
-  if (p.parts > 1 && first >= tiles) return;  // (uniform; the ranges are counted alike in the combine)
+  int first = 0, tiles = causal_tiles(p, w, G, items);
+  if constexpr (SPLIT) {
+    const int per = causal_range(tiles, p.parts);
+    first = part * per;
+    tiles = min(tiles, first + per);
+    if (first >= tiles) return;  // (uniform; the ranges are counted alike in the combine)
+  }
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&smem[0][0];
   auto issue = [&](int t) {
     const size_t blk = ((size_t)p.page_table[t] * p.Hkv + g) * (DTREE_PAGE * D);
@@ -331,7 +337,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void causal_attn_kernel(Caus
   }
   if (item >= items) return;
   const float l = l_run + __shfl_xor(l_run, 32);
-  if (p.parts > 1) {
+  if constexpr (SPLIT) {
     const size_t u = ((size_t)(part * nw + w) * p.Hkv + g) * 4 + wave;
     f32x4_t* po = reinterpret_cast<f32x4_t*>(p.part + u * (32 * D)) + lane;
 #pragma unroll
@@ -409,8 +415,12 @@ constexpr int kFill = 256;
 // Workspace of one key range of every workgroup.
 size_t causal_part_bytes(int D, int groups) { return (size_t)groups * 4 * (32 * D + 64) * sizeof(float); }
 
-int causal_parts(int groups, int past, int n) {
+// Ranges pay once they save more than the second kernel costs, about 5 us: two
+// pages' walk at head_dim 256 (4.5 us a page; 5 pages, 300 rows: 52 -> 40 us),
+// four at 128 (2.1 us; 13 pages, 300 rows: 40 -> 35, but 5 pages 24.5 -> 27.8).
+int causal_parts(int D, int groups, int past, int n) {
   const int pages = (past + n + DTREE_PAGE - 1) / DTREE_PAGE;
+  if (pages < (D == 128 ? 8 : 4)) return 1;
   return std::max(1, std::min(kFill / groups, pages / kMinRange));
 }
 
@@ -474,7 +484,7 @@ extern "C" int dtree_causal_attention_split(const DtreeAttnArgs* a, int32_t past
   p.Hq = a->num_heads; p.Hkv = a->num_kv_heads; p.past = past_length; p.n = num_rows; p.rows = a->rows_padded;
   p.scale_log2 = a->scale * 1.4426950408889634f;
   const int live = causal_groups(G * ((num_rows + 31) / 32)) * p.Hkv;
-  p.parts = causal_parts(live, past_length, num_rows);
+  p.parts = causal_parts(D, live, past_length, num_rows);
   // without room for two ranges, one: the kernel then needs no workspace
   const size_t fit = workspace && ((uintptr_t)workspace & 15) == 0 ? workspace_bytes / causal_part_bytes(D, live) : 0;
   if ((size_t)p.parts > fit) p.parts = std::max(1, (int)fit);
@@ -487,12 +497,14 @@ extern "C" int dtree_causal_attention_split(const DtreeAttnArgs* a, int32_t past
   if (D == 128) {
     causal_append_kernel<128, 128><<<agrid, 256, 0, stream>>>(p);
     DTREE_LAUNCH_CHECK("causal_attention append launch");
-    causal_attn_kernel<128, 128, false><<<grid, 256, 0, stream>>>(p);
+    if (p.parts == 1) causal_attn_kernel<128, 128, false, false><<<grid, 256, 0, stream>>>(p);
+    else causal_attn_kernel<128, 128, false, true><<<grid, 256, 0, stream>>>(p);
     if (p.parts > 1) causal_combine_kernel<128, false><<<cgrid, 256, 0, stream>>>(p);
   } else {
     causal_append_kernel<256, 64><<<agrid, 256, 0, stream>>>(p);
     DTREE_LAUNCH_CHECK("causal_attention append launch");
-    causal_attn_kernel<256, 64, true><<<grid, 256, 0, stream>>>(p);
+    if (p.parts == 1) causal_attn_kernel<256, 64, true, false><<<grid, 256, 0, stream>>>(p);
+    else causal_attn_kernel<256, 64, true, true><<<grid, 256, 0, stream>>>(p);
     if (p.parts > 1) causal_combine_kernel<256, true><<<cgrid, 256, 0, stream>>>(p);
   }
   DTREE_LAUNCH_CHECK("causal_attention launch");

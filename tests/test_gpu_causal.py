@@ -116,12 +116,15 @@ def _range_bytes(Hq, Hkv, D, n):
 
 
 @pytest.mark.parametrize("geo,D", [("qwen3", 128), ("gated", 256)])
-@pytest.mark.parametrize("past,n", [(300, 1), (0, 200), (1000, 31), (4095, 33), (1985, 130), (127, 513)])
+@pytest.mark.parametrize("past,n", [(300, 1), (0, 200), (448, 64), (383, 66), (1000, 31), (4095, 33), (1985, 130),
+                                    (127, 513)])
 def test_causal_key_ranges(gpu_device, geo, D, past, n):
     """Prefixes that end inside a page, rows whose first keys lie past some
     ranges, empty last ranges; pages the segment does not own hold NaN."""
     full = N.lib().dtree_causal_attention_workspace_bytes(D)
-    assert _case(gpu_device, geo, 8, 2, past, n, workspace=(full, 0)) > 0
+    pages = (past + n + 63) // 64
+    used = _case(gpu_device, geo, 8, 2, past, n, workspace=(full, 0))
+    assert (used > 0) == (pages >= (8 if D == 128 else 4))
 
 
 @pytest.mark.parametrize("geo,D,Hq,Hkv", [("qwen3", 128, 12, 3), ("qwen3", 128, 16, 2), ("gated", 256, 10, 5)])
