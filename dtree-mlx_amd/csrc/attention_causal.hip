@@ -55,8 +55,9 @@ struct CausalParams {
 // each; `items` pairs per group.
 __host__ __device__ __forceinline__ int causal_groups(int items) { return (items + 3) / 4; }
 
-// Pages that workgroup w's rows need.
+// Pages that workgroup w's rows need (none: it has padding rows alone).
 __device__ __forceinline__ int causal_tiles(const CausalParams& p, int w, int G, int items) {
+  if (32 * (4 * w / G) >= p.n) return 0;
   const int rbl = min(4 * w + 3, items - 1) / G;  // the workgroup's last row block
   return (min(p.past + 32 * (rbl + 1), p.past + p.n) + DTREE_PAGE - 1) / DTREE_PAGE;
 }
@@ -214,7 +215,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void causal_attn_kernel(Caus
 #pragma unroll
     for (int i = 0; i < PW / 2; ++i) lds_load16(vr, wave * (PW * 512) + 1024 * i + 16 * lane, lds + PB + 1024 * i);
   };
-  issue(first);
+  if (first < tiles) issue(first);
   // This lane's dims 16 j + 8 h .. + 7 of its query row: q_norm, RoPE (pairs j,
   // j + R / 32 in one lane), softmax scale in log2 units, split.
   u32x4_t qh[NJ], ql[NJ];

@@ -159,6 +159,14 @@ def test_causal_group_sizes(gpu_device, geo, Hq, Hkv):
     _case(gpu_device, geo, Hq, Hkv, 70, 161, tiled=False)
 
 
+@pytest.mark.parametrize("geo,Hq,Hkv", [("qwen3", 4, 1), ("qwen3", 16, 2), ("gated", 4, 2)])
+@pytest.mark.parametrize("past,n", [(0, 1), (130, 33), (64, 128), (70, 129)])
+def test_causal_padding_workgroups(gpu_device, geo, Hq, Hkv, past, n):
+    """Rows padded to 256: workgroups of padding rows alone write zeros (and
+    read no page of the cache)."""
+    _case(gpu_device, geo, Hq, Hkv, past, n, pad=256)
+
+
 @pytest.mark.parametrize("geo", ["qwen3", "gated"])
 def test_causal_without_norms(gpu_device, geo):
     _case(gpu_device, geo, 4, 2, 5, 40, norms=False)
