@@ -16,7 +16,7 @@ __device__ __forceinline__ void lds_load16(u32x4_t r, unsigned off, unsigned lds
   const s32x4_t rsrc = s32x4_t{uni(r[0]), uni(r[1]), uni(r[2]), uni(r[3])};
   const int lds = uni(lds_addr);
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(lds), "v"(off), "s"(rsrc) : "memory");
+               :: "s"(lds), "v"(off), "s"(rsrc) : "m0", "memory");
 }
 
 // The same for a resource and an LDS address that are in scalar registers.
@@ -25,7 +25,7 @@ __device__ __forceinline__ void lds_load16_s(uint32_t base_lo, uint32_t base_hi,
   typedef uint32_t s32x4_t __attribute__((ext_vector_type(4)));
   const s32x4_t rsrc = s32x4_t{base_lo, base_hi, size, 0x00020000u};
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(lds_addr), "v"(off), "s"(rsrc) : "memory");
+               :: "s"(lds_addr), "v"(off), "s"(rsrc) : "m0", "memory");
 }
 
 // This wave's loads but the N youngest have landed and its LDS reads are done;

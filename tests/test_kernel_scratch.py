@@ -1,10 +1,14 @@
-"""Kernels of the built library that keep per-lane values in scratch memory.
+"""Properties of the pipelined kernels' code that no result shows.
 
-The pipelined kernels order their direct loads by counting outstanding memory
+Scratch: the pipelined kernels order their direct loads by counting outstanding memory
 operations; the compiler does not know of those loads, so a scratch access
 inside such a loop also waits for all of them (measured: the pair layout's
-long GEMM ran 4 to 5 times as slow). The code objects' own metadata says what
-each kernel uses."""
+long GEMM ran 3 to 5 times as slow). The code objects' own metadata says what
+each kernel uses.
+
+m0: an asm block that writes it names it as clobbered, or the compiler may keep
+a value of its own there across the block."""
+import re
 import struct
 
 import msgpack
@@ -54,3 +58,12 @@ def test_pipelined_kernels_use_no_scratch():
     pipelined = [k for k in kernels if any(n in k[".name"] for n in ("long_kernel", "longq_kernel", "causal_attn"))]
     assert len(pipelined) >= 50, [k[".name"] for k in kernels]
     assert [k[".name"] for k in pipelined if k[".private_segment_fixed_size"]] == []
+
+
+def test_asm_that_writes_m0_names_it():
+    blocks = []
+    for f in sorted((N.LIB_PATH.parent.parent / "csrc").glob("*.h*")):
+        blocks += [(f.name, b) for b in re.findall(r"\basm\b[^;]*?\(.*?\);", f.read_text(), re.S)
+                   if re.search(r"\b(s_mov_b32|v_readfirstlane_b32|s_add_u32)\s+m0\b", b)]
+    assert len(blocks) >= 2
+    assert [f for f, b in blocks if '"m0"' not in b.rsplit(":", 1)[1]] == []
