@@ -242,7 +242,8 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void causal_attn_kernel(Caus
       const float rs = rsqrtf(ss * (1.0f / D) + p.eps);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const u32x4_t nwv = ld_u32x4(p.q_norm + 16 * j + 8 * h);
+        u32x4_t nwv;  // (a weight at any 2-byte address, as the tree kernels take it)
+        __builtin_memcpy(&nwv, p.q_norm + 16 * j + 8 * h, sizeof(nwv));
 #pragma unroll
         for (int i = 0; i < 8; ++i)
           q[j][i] *= rs * __uint_as_float((i & 1) ? (nwv[i >> 1] & 0xffff0000u) : (nwv[i >> 1] << 16));
@@ -465,8 +466,8 @@ extern "C" int dtree_causal_attention_split(const DtreeAttnArgs* a, int32_t past
   const int width = a->num_heads * qs + 2 * a->num_kv_heads * D;
   DTREE_REQUIRE(a->ld_qkv >= width && a->ld_qkv % 4 == 0 && ((uintptr_t)a->qkv & 15) == 0,
                 "causal_attention: qkv rows of [q | k | v] heads, 16-byte aligned");
-  DTREE_REQUIRE(((uintptr_t)a->q_norm & 15) == 0 && ((uintptr_t)a->k_pages & 15) == 0 && ((uintptr_t)a->v_pages & 15) == 0,
-                "causal_attention: q_norm and the pages must be 16-byte aligned");
+  DTREE_REQUIRE(((uintptr_t)a->k_pages & 15) == 0 && ((uintptr_t)a->v_pages & 15) == 0,
+                "causal_attention: the pages must be 16-byte aligned");
   const int od = a->num_heads * D;
   DTREE_REQUIRE(((uintptr_t)a->out & 7) == 0 && ((uintptr_t)a->out_lo & 7) == 0 &&
                     (a->out_layout == DTREE_W_ROWMAJOR ? a->ld_out >= od && a->ld_out % 4 == 0

@@ -10,6 +10,11 @@ namespace dtree {
 // loads; the stage waits below do it by count. The load has no register
 // result, and the callers wait for it before its LDS is read or released.
 // s_nop 4 covers m0 and a resource word that a VALU lane read has just written.
+// m0 is named as clobbered, so that a value the compiler puts there is made again
+// after the block; its warning about reserved registers means that the block
+// does not preserve it, which is what is said here.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ int uni(uint32_t v) { return __builtin_amdgcn_readfirstlane((int)v); }
 __device__ __forceinline__ void lds_load16(u32x4_t r, unsigned off, unsigned lds_addr) {
   typedef int s32x4_t __attribute__((ext_vector_type(4)));
@@ -27,6 +32,8 @@ __device__ __forceinline__ void lds_load16_s(uint32_t base_lo, uint32_t base_hi,
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                :: "s"(lds_addr), "v"(off), "s"(rsrc) : "m0", "memory");
 }
+
+#pragma clang diagnostic pop
 
 // This wave's loads but the N youngest have landed and its LDS reads are done;
 // then the workgroup barrier.

@@ -370,7 +370,7 @@ int dtree_embed_tokens(const int32_t* tokens, int32_t n, const uint16_t* embed, 
  * up to its own. Arguments as for dtree_tree_attention, with qkv, out and the
  * RoPE tables of rows_padded rows (a multiple of 32; rows >= num_rows of out
  * become zero); desc, max_past_length, write_cache and the workspace are not
- * used. q_norm and the pages are 16-byte aligned. dtree_rope_positions fills
+ * used. The pages are 16-byte aligned. dtree_rope_positions fills
  * such tables ([rows][rope_dims / 2]) for positions first_position + row, as
  * dtree_rope_table does for a tree's positions.
  */

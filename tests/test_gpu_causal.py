@@ -28,7 +28,7 @@ def _rope(x, pos, dims, base):
     return torch.cat([a * c - b * s, a * s + b * c, x[..., dims:]], -1)
 
 
-def _case(dev, geo, Hq, Hkv, past, n, tiled=True, norms=True, workspace=None, pad=32):
+def _case(dev, geo, Hq, Hkv, past, n, tiled=True, norms=True, workspace=None, pad=32, norm_off=0):
     """workspace: None, or (bytes, misalignment) for dtree_causal_attention_split;
     returns the share of the workspace that the call wrote. pad: rows of qkv and
     out come in multiples of it."""
@@ -41,7 +41,7 @@ def _case(dev, geo, Hq, Hkv, past, n, tiled=True, norms=True, workspace=None, pa
     ld = Hq * qs + 2 * Hkv * D
     qkv = torch.zeros(rows, ld, device=dev)
     qkv[:n] = rnd(n, ld)
-    qn, kn = ((1 + 0.1 * rnd(D)).to(torch.bfloat16) for _ in range(2))
+    qn, kn = ((1 + 0.1 * rnd(D + norm_off)).to(torch.bfloat16)[norm_off:] for _ in range(2))
     npages = (past + n + 63) // 64 + 2
     cache = PagedKVCache(1, Hkv, D, 64 * npages, device=dev,
                          page_order=torch.randperm(npages, generator=torch.Generator().manual_seed(n)))
@@ -170,6 +170,11 @@ def test_causal_padding_workgroups(gpu_device, geo, Hq, Hkv, past, n):
 @pytest.mark.parametrize("geo", ["qwen3", "gated"])
 def test_causal_without_norms(gpu_device, geo):
     _case(gpu_device, geo, 4, 2, 5, 40, norms=False)
+
+
+@pytest.mark.parametrize("geo", ["qwen3", "gated"])
+def test_causal_norms_at_odd_addresses(gpu_device, geo):
+    _case(gpu_device, geo, 4, 2, 5, 40, norm_off=1)
 
 
 def test_causal_rejects_bad_shapes(gpu_device):
