@@ -152,18 +152,25 @@ Q4_SHAPES = [(128, 256, 640), (128, 512, 512), (384, 19456, 320), (640, 19520, 5
 
 @pytest.mark.parametrize("rows,n,k", Q4_SHAPES)
 @pytest.mark.parametrize("lo", [False, True])
-def test_long_q4_tiles_match_float64(gpu_device, rows, n, k, lo):
+@pytest.mark.parametrize("mean", [0.0, 4.0])
+def test_long_q4_tiles_match_float64(gpu_device, rows, n, k, lo, mean):
     """fp32 store; weights with a constant-group (scale 0) row block and a group
-    whose bias dwarfs its scale. The group sums are exact products of bf16
-    values accumulated in fp32 and the bias term carries 24 bits, so the error
-    stays within k 2^-23 of sum |x| (|s| 143 + |b|)."""
+    whose bias dwarfs its scale; activations with and without a mean. The group
+    sums are exact products of bf16 values, at most 31 |s| per unit of |x|,
+    accumulated in fp32, and the bias term carries 24 bits, so the error stays
+    within k 2^-23 of sum |x| (|s| 31 + |b|). Its norm: a rounding of the
+    accumulator is 0.29 * 2^-24 of it at random, there are k / 64 of them, and
+    its rms is that of up to eight groups of 16 + q, (16 + 7.5) / 4.6 times the
+    result's share of eight groups: 5.1 sqrt(8) 0.29 2^-24 = 2.5e-7 of the
+    result, and as much again at the most for the sums inside the groups and the
+    result itself. (Nibbles as 128 + q gave 4.4e-7 to 1.6e-6.)"""
     g = torch.Generator(device=gpu_device)
     g.manual_seed(rows + n + k)
     wq, sc, bi = q4_random_mlx(n, k, g, gpu_device)
     sc[:32, 0] = 0.0
     bi[32:64, 1] = 40.0
     lin = Q4Linear(*q4_to_tiled(wq, sc, bi))
-    xf = torch.empty(rows, k, device=gpu_device).normal_(generator=g)
+    xf = torch.empty(rows, k, device=gpu_device).normal_(mean, 1.0, generator=g)
     hi = xf.to(torch.bfloat16)
     low = (xf - hi.float()).to(torch.bfloat16)
     xt, xlt = tile_weight(hi), tile_weight(low)
@@ -175,13 +182,16 @@ def test_long_q4_tiles_match_float64(gpu_device, rows, n, k, lo):
     a.w = lin.words.data_ptr(); a.w_scales = lin.sb.data_ptr(); a.w_layout = N.W_Q4G64; a.n = n; a.k = k
     a.epilogue = N.EPI_STORE_F32; a.out_f32 = out.data_ptr(); a.ld_out_f32 = n
     a.ss_in = ss.data_ptr(); a.ss_tiles = k // 32; a.norm_dim = k; a.eps = 1e-6
-    print(f"q4 gemm_long rows={rows} n={n} k={k} lo={lo}", flush=True)
+    print(f"q4 gemm_long rows={rows} n={n} k={k} lo={lo} mean={mean}", flush=True)
     N.check(N.lib().dtree_gemm_long(C.byref(a), torch.cuda.current_stream().cuda_stream), "gemm_long")
     torch.cuda.synchronize()
     rs = torch.rsqrt(ss.double().transpose(1, 2).reshape(rows, -1).sum(1) / k + 1e-6)
     x = hi.double() + (low.double() if lo else 0.0)
     ref = (x @ q4_dequant(lin).double().T) * rs[:, None]
-    mag = (x.abs() @ (143.0 * sc.double().abs() + bi.double().abs()).repeat_interleave(64, 1).T) * rs[:, None]
+    mag = (x.abs() @ (31.0 * sc.double().abs() + bi.double().abs()).repeat_interleave(64, 1).T) * rs[:, None]
     assert ((out.double() - ref).abs() <= k * 2.0 ** -23 * mag).all()
-    rel = ((out.double() - ref).norm() / ref.norm()).item()
-    assert rel <= 2e-6, rel  # fp32 sums: measured 3e-7
+    # (without the columns of the large bias, whose results would hide the others')
+    keep = torch.arange(n, device=gpu_device) // 32 != 1
+    rel = ((out.double() - ref)[:, keep].norm() / ref[:, keep].norm()).item()
+    print(f"relative error {rel:.2e}", flush=True)
+    assert rel <= 4e-7, rel  # measured below 3e-7
