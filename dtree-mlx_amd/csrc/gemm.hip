@@ -2112,6 +2112,12 @@ extern "C" int dtree_gemm_long(const DtreeGemmArgs* a, hipStream_t stream) {
   return q4 ? launch_long_q4(l, epi, device_cus(), stream) : launch_long_dense(l, epi, h16, device_cus(), stream);
 }
 
+extern "C" int dtree_gemm_long_tile(const DtreeGemmArgs* a) {
+  DTREE_REQUIRE(a && a->rows_padded > 0 && a->n > 0 && a->k > 0, "gemm_long_tile: args");
+  return long_tile(a->w_layout == DTREE_W_Q4G64, a->w_layout == DTREE_W_TILED_F16, a->x_lo != nullptr, a->epilogue,
+                   a->rows_padded, a->n, a->k, device_cus());
+}
+
 extern "C" size_t dtree_lmhead_candidates_bytes(int32_t rows_padded) {
   return (size_t)1024 * rows_padded * sizeof(int2);
 }

@@ -22,5 +22,7 @@ struct LongParams {
 // tiles are filled in here.
 int launch_long_dense(LongParams p, int epi, bool h16, int cus, hipStream_t st);
 int launch_long_q4(LongParams p, int epi, int cus, hipStream_t st);
+// The tile the launches above choose, 1000 rows + columns.
+int long_tile(bool q4, bool h16, bool lo, int epi, int rows, int n, int k, int cus);
 
 }  // namespace dtree

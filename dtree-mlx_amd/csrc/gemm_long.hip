@@ -811,10 +811,25 @@ int pick_tile(const TileCost* cost, int from, int count, int rows, int n, int cu
 
 }  // namespace
 
+namespace {
+int dense_tile(int epi, int rows, int n, int cus) {
+  return pick_tile(kTileCost, 0, epi == DTREE_EPI_RESIDUAL ? kT256x320 : kTiles, rows, n, cus);
+}
+int q4_tile(int rows, int n, int k, int cus) {
+  return pick_tile(kQTileCost, k % 128 ? kQ128x256 : kQ128x128, kQTiles, rows, n, cus);
+}
+}  // namespace
+
+int long_tile(bool q4, bool h16, bool lo, int epi, int rows, int n, int k, int cus) {
+  if (q4 ? lo : !h16) return 1000 * 128 + 128;
+  const TileCost& c = q4 ? kQTileCost[q4_tile(rows, n, k, cus)] : kTileCost[dense_tile(epi, rows, n, cus)];
+  return 1000 * c.tm + c.tn;
+}
+
 int launch_long_dense(LongParams p, int epi, bool h16, int cus, hipStream_t st) {
   if (!h16)
     return p.x_lo ? launch_tile<T128x128, kBf16Lo>(p, epi, st) : launch_tile<T128x128, kBf16>(p, epi, st);
-  switch (pick_tile(kTileCost, 0, epi == DTREE_EPI_RESIDUAL ? kT256x320 : kTiles, p.rows, p.n, cus)) {
+  switch (dense_tile(epi, p.rows, p.n, cus)) {
     case kT64x64: return launch_tile<T64x64k, kF16>(p, epi, st);
     case kT64x128: return launch_tile<T64x128k, kF16>(p, epi, st);
     case kT256x128: return launch_tile<T256x128, kF16>(p, epi, st);
@@ -828,7 +843,7 @@ int launch_long_dense(LongParams p, int epi, bool h16, int cus, hipStream_t st) 
 
 int launch_long_q4(LongParams p, int epi, int cus, hipStream_t st) {
   if (p.x_lo) return launch_tile<Q128x128lo, kQ4Lo>(p, epi, st);
-  switch (pick_tile(kQTileCost, p.k % 128 ? kQ128x256 : kQ128x128, kQTiles, p.rows, p.n, cus)) {
+  switch (q4_tile(p.rows, p.n, p.k, cus)) {
     case kQ128x256: return launch_tile<Q128x256, kQ4>(p, epi, st);
     case kQ256x192: return launch_tile<Q256x192, kQ4>(p, epi, st);
     case kQ256x256: return launch_tile<Q256x256, kQ4>(p, epi, st);

@@ -356,6 +356,9 @@ int dtree_rownorm(const float* x, int32_t ldx, int32_t rows_padded, int32_t hidd
  * (rows n .. rows_padded - 1 zero), without the RoPE table.
  */
 int dtree_gemm_long(const DtreeGemmArgs* args, hipStream_t stream);
+/* The output tile dtree_gemm_long takes for these arguments (rows_padded, n, k,
+ * epilogue, w_layout, x_lo set or not): 1000 * rows + columns. Host only. */
+int dtree_gemm_long_tile(const DtreeGemmArgs* args);
 int dtree_embed_tokens(const int32_t* tokens, int32_t n, const uint16_t* embed, int32_t embed_layout,
                        const uint16_t* embed_scales, int32_t vocab, int32_t hidden, const uint16_t* norm_w,
                        int32_t rows_padded, float* x, uint16_t* xg, uint16_t* xg_lo, int32_t xg_layout, float* ss,

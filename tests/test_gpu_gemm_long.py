@@ -1,9 +1,10 @@
 """dtree_gemm_long's tile shapes against a float64 product.
 
-The fp16 path picks one of eight tile shapes by rows and columns; the cases
-below reach every one of them, with ragged last row and column tiles, with
-fewer K stages than the pipeline holds, and with outputs too misaligned for
-the vector stores. Bounds: the fp32 accumulation of K products differs from
+The fp16 path picks one of eight tile shapes by rows and columns, the q4 path
+one of four; each case names the tile it is for, which the library has to
+confirm, and test_every_tile_has_a_case that none is left out: with ragged last
+row and column tiles, with fewer K stages than the pipeline holds, and with
+outputs too misaligned for the vector stores. Bounds: the fp32 accumulation of K products differs from
 the exact sum by at most K 2^-24 sum |x w| (checked in the result's units);
 fp16 and bf16 outputs add their own rounding (2^-11, 2^-8 relative)."""
 import ctypes as C
@@ -21,19 +22,27 @@ def _silu(t):
     return t * torch.sigmoid(t)
 
 
-def _long(dev, rows, n, k, epi, misaligned=False, seed=0, form="f16"):
+def _tile(rows, n, k, epi, w_layout, pair=False):
+    a = N.GemmArgs()
+    a.rows_padded, a.n, a.k, a.epilogue, a.w_layout, a.x_lo = rows, n, k, epi, w_layout, 16 if pair else None
+    t = N.lib().dtree_gemm_long_tile(C.byref(a))
+    return t // 1000, t % 1000
+
+
+def _long(dev, rows, n, k, epi, misaligned=False, seed=0, form="f16", tile=None):
     """form: fp16 operands, bf16 operands, or bf16 weights with the activations
-    and the outputs as split pairs of bf16 planes (value = hi + lo)."""
+    and the outputs as split pairs of bf16 planes (value = hi + lo); q4 weights
+    with bf16 activations."""
     g = torch.Generator(device=dev)
     g.manual_seed(seed + rows + 3 * n + 7 * k)
-    h16, pair = form == "f16", form == "pair"
+    h16, pair, q4 = form == "f16", form == "pair", form == "q4"
     dt = torch.float16 if h16 else torch.bfloat16
     x = torch.empty(rows, k, device=dev).normal_(generator=g)
     xl = (x - x.to(dt).float()).to(dt)
     x = x.to(dt)
     w = torch.empty(n, k, device=dev).normal_(0.0, 0.05, generator=g).to(dt)
-    tile = tile_weight_f16 if h16 else tile_weight
-    xt, xlt, wt = tile(x), tile(xl), tile(w)
+    to_tiles = tile_weight_f16 if h16 else tile_weight
+    xt, xlt, wt = to_tiles(x), to_tiles(xl), to_tiles(w)
     layout = N.W_TILED_F16 if h16 else N.W_TILED
     off = 1 if misaligned else 0  # rows of odd length from an odd element: no vector access is aligned
     width = n // 2 if epi == N.EPI_SWIGLU else n
@@ -43,6 +52,13 @@ def _long(dev, rows, n, k, epi, misaligned=False, seed=0, form="f16"):
     if pair:
         a.x_lo = xlt.data_ptr()
         x = x.double() + xl.double()
+    if q4:
+        wq, sc, bi = q4_random_mlx(n, k, g, dev)
+        lin = Q4Linear(*q4_to_tiled(wq, sc, bi))
+        a.w, a.w_scales, a.w_layout = lin.words.data_ptr(), lin.sb.data_ptr(), N.W_Q4G64
+        w = q4_dequant(lin)
+    if tile is not None:
+        assert _tile(rows, n, k, epi, a.w_layout, pair) == tile
     a.ldx = k; a.rows_padded = rows; a.n = n; a.k = k; a.epilogue = epi
     a.norm_dim = k; a.eps = 1e-6
     a.out_layout = N.W_ROWMAJOR if misaligned else layout
@@ -68,7 +84,9 @@ def _long(dev, rows, n, k, epi, misaligned=False, seed=0, form="f16"):
     N.check(N.lib().dtree_gemm_long(C.byref(a), torch.cuda.current_stream().cuda_stream), "gemm_long")
     torch.cuda.synchronize()
     acc = x.double() @ w.double().T
-    bound = (x.double().abs() @ w.double().abs().T).max().item() * k * 2.0 ** -24 * rs.max().item() + 1e-6
+    # (q4: the bias term stands apart from the group sums, on values up to 31 |s|)
+    mag = (31 * sc.double().abs() + bi.double().abs()).repeat_interleave(64, 1) * 2 if q4 else w.double().abs()
+    bound = (x.double().abs() @ mag.T).max().item() * k * 2.0 ** -24 * rs.max().item() + 1e-6
     f = f32[off:].view(rows, n + off)[:, :n].double()
     if misaligned:  # row-major bf16
         b = sum(t[off:].view(rows, ld)[:, :width].view(torch.bfloat16).double() for t in (act, actl))
@@ -99,15 +117,24 @@ def _long(dev, rows, n, k, epi, misaligned=False, seed=0, form="f16"):
         torch.testing.assert_close(sso.double(), want, rtol=1e-5, atol=1e-5)
 
 
-# (rows, n): 128x128 (K halves), 256x128, 256x192, 256x256, 256x320, 256x384 tiles
-SHAPES = [(128, 256), (1152, 6144), (640, 19456), (1152, 12416), (1024, 19456), (1152, 24576)]
+# (rows, n, tile, tile with the residual epilogue, which the two widest do not take)
+SHAPES = [(128, 256, (64, 64), (64, 64)), (128, 6144, (64, 64), (64, 64)), (384, 2560, (64, 64), (64, 64)),
+          (640, 2432, (64, 128), (64, 128)), (256, 6144, (64, 128), (64, 128)),
+          (896, 2432, (128, 128), (128, 128)), (256, 12288, (128, 128), (128, 128)),
+          (384, 12288, (256, 128), (256, 128)), (768, 6144, (256, 128), (256, 128)),
+          (384, 19456, (256, 192), (256, 192)), (768, 12288, (256, 192), (256, 192)),
+          (640, 19456, (256, 256), (256, 256)), (896, 12416, (256, 256), (256, 256)),
+          (384, 6144, (128, 128), (128, 128)), (768, 2560, (64, 128), (64, 128)),
+          (1152, 6144, (256, 128), (256, 128)), (1152, 12416, (256, 256), (256, 256)), (1152, 24576, (256, 256), (256, 256)),
+          (640, 24576, (256, 320), (256, 192)), (1024, 19456, (256, 320), (256, 192)),
+          (1152, 19456, (256, 384), (256, 192)), (1024, 24576, (256, 384), (256, 192))]
 
 
-@pytest.mark.parametrize("rows,n", SHAPES)
+@pytest.mark.parametrize("rows,n,tile,tile_res", SHAPES)
 @pytest.mark.parametrize("epi", [N.EPI_STORE_F32, N.EPI_RESIDUAL, N.EPI_SWIGLU, N.EPI_STORE_BF16])
 @pytest.mark.parametrize("k", [64, 320])
-def test_long_tiles_match_float64(gpu_device, rows, n, epi, k):
-    _long(gpu_device, rows, n, k, epi)
+def test_long_tiles_match_float64(gpu_device, rows, n, tile, tile_res, epi, k):
+    _long(gpu_device, rows, n, k, epi, tile=tile_res if epi == N.EPI_RESIDUAL else tile)
 
 
 # bf16 weights, with one and two activation planes: 128x128 tiles, several per
@@ -125,35 +152,49 @@ def test_long_bf16_64_column_tail(gpu_device, form):
     _long(gpu_device, 256, 448, 192, N.EPI_STORE_F32, form=form)
 
 
-# short prompts: 64x64, 64x128 and 128x128 tiles, in one and two per CU
-@pytest.mark.parametrize("rows,n", [(128, 6144), (384, 2560), (256, 12288), (768, 2560), (896, 2432), (384, 6144)])
-@pytest.mark.parametrize("epi", [N.EPI_STORE_F32, N.EPI_RESIDUAL, N.EPI_SWIGLU, N.EPI_STORE_BF16])
-def test_long_small_tiles(gpu_device, rows, n, epi):
-    _long(gpu_device, rows, n, 192, epi)
+TAILS = [(128, 64, (64, 64)), (128, 12352, (64, 128)), (640, 4160, (128, 128)), (384, 12352, (256, 128)),
+         (384, 16448, (256, 192)), (1024, 12352, (256, 256)), (640, 21824, (256, 320)), (1152, 19520, (256, 384)), (640, 19520, (256, 256)),
+         (1024, 19520, (256, 320)), (1152, 24640, (256, 256))]
 
 
-@pytest.mark.parametrize("rows,n", [(128, 64), (128, 12352), (1024, 12352), (640, 19520), (1024, 19520), (1152, 24640)])
-def test_long_tiles_64_column_tail(gpu_device, rows, n):
-    _long(gpu_device, rows, n, 192, N.EPI_STORE_F32)
+@pytest.mark.parametrize("rows,n,tile", TAILS)
+def test_long_tiles_64_column_tail(gpu_device, rows, n, tile):
+    _long(gpu_device, rows, n, 192, N.EPI_STORE_F32, tile=tile)
 
 
-@pytest.mark.parametrize("rows,n", [(384, 256), (1152, 6144), (1024, 19456)])
+@pytest.mark.parametrize("rows,n", [(384, 256), (1152, 6144), (1024, 19456), (1152, 19456)])
 @pytest.mark.parametrize("epi", [N.EPI_STORE_F32, N.EPI_RESIDUAL, N.EPI_SWIGLU, N.EPI_STORE_BF16])
 def test_long_tiles_misaligned_outputs(gpu_device, rows, n, epi):
     _long(gpu_device, rows, n, 128, epi, misaligned=True)
 
 
-# 128x128 (K halves), 128x256 (k % 128 != 0 or wide), 256x192, 256x256 tiles; a
-# K of 5, 8 and 19 groups ends inside, at and past the eight groups of a
-# correction step
-Q4_SHAPES = [(128, 256, 640), (128, 512, 512), (384, 19456, 320), (640, 19520, 576), (1152, 12352, 512),
-             (1152, 12352, 1216), (256, 320, 1216)]
+# Ragged last row and column tiles; k % 128 != 0 keeps to the three wider tiles.
+# A K of 5, 8, 9 and 19 groups ends inside, at and past the eight groups of a
+# correction step.
+Q4_SHAPES = [(128, 256, 640, (128, 128)), (128, 512, 512, (128, 128)), (384, 384, 1152, (128, 128)),
+             (384, 12416, 512, (128, 256)), (128, 256, 320, (128, 256)), (256, 384, 1216, (128, 256)),
+             (1152, 9728, 512, (256, 192)), (384, 24576, 576, (256, 192)),
+             (384, 19456, 320, (128, 256)), (640, 19456, 576, (256, 256)), (1152, 12416, 1152, (256, 256))]
+Q4_TAILS = [(640, 19520, 576, (256, 256)), (1152, 12352, 512, (256, 256)),
+            (256, 320, 1216, (128, 256)), (384, 21824, 512, (256, 192)), (1152, 12352, 1216, (256, 256))]
 
 
-@pytest.mark.parametrize("rows,n,k", Q4_SHAPES)
+@pytest.mark.parametrize("rows,n,k,tile", Q4_SHAPES)
+@pytest.mark.parametrize("epi", [N.EPI_RESIDUAL, N.EPI_SWIGLU, N.EPI_STORE_BF16])
+def test_long_q4_epilogues(gpu_device, rows, n, k, tile, epi):
+    _long(gpu_device, rows, n, k, epi, form="q4", tile=tile)
+
+
+@pytest.mark.parametrize("rows,n", [(256, 384), (1152, 9728)])
+@pytest.mark.parametrize("epi", [N.EPI_STORE_F32, N.EPI_RESIDUAL, N.EPI_SWIGLU, N.EPI_STORE_BF16])
+def test_long_q4_misaligned_outputs(gpu_device, rows, n, epi):
+    _long(gpu_device, rows, n, 320, epi, misaligned=True, form="q4")
+
+
+@pytest.mark.parametrize("rows,n,k,tile", Q4_SHAPES + Q4_TAILS)
 @pytest.mark.parametrize("lo", [False, True])
 @pytest.mark.parametrize("mean", [0.0, 4.0])
-def test_long_q4_tiles_match_float64(gpu_device, rows, n, k, lo, mean):
+def test_long_q4_tiles_match_float64(gpu_device, rows, n, k, tile, lo, mean):
     """fp32 store; weights with a constant-group (scale 0) row block and a group
     whose bias dwarfs its scale; activations with and without a mean. The group
     sums are exact products of bf16 values, at most 31 |s| per unit of |x|,
@@ -182,6 +223,7 @@ def test_long_q4_tiles_match_float64(gpu_device, rows, n, k, lo, mean):
     a.w = lin.words.data_ptr(); a.w_scales = lin.sb.data_ptr(); a.w_layout = N.W_Q4G64; a.n = n; a.k = k
     a.epilogue = N.EPI_STORE_F32; a.out_f32 = out.data_ptr(); a.ld_out_f32 = n
     a.ss_in = ss.data_ptr(); a.ss_tiles = k // 32; a.norm_dim = k; a.eps = 1e-6
+    assert _tile(rows, n, k, N.EPI_STORE_F32, N.W_Q4G64, lo) == ((128, 128) if lo else tile)
     print(f"q4 gemm_long rows={rows} n={n} k={k} lo={lo} mean={mean}", flush=True)
     N.check(N.lib().dtree_gemm_long(C.byref(a), torch.cuda.current_stream().cuda_stream), "gemm_long")
     torch.cuda.synchronize()
