@@ -313,6 +313,20 @@ class TreeEngineBase:
     # under 2 GB for the 9B shape.
     PREFILL_SEGMENT = 4096
 
+    def _prefill_segment(self, tokens: int) -> int:
+        """Rows per pass of a prompt, with the buffers for them allocated:
+        PREFILL_SEGMENT, or, where the device has no room for that many, half of
+        it and so on down to 1024."""
+        seg = self.PREFILL_SEGMENT
+        while True:
+            try:
+                self._prefill_buffers(min(seg, 128 * ((tokens + 127) // 128)))
+                return seg
+            except torch.cuda.OutOfMemoryError:
+                if seg <= 1024:
+                    raise
+                seg = max(1024, seg // 256 * 128)
+
     def _long_gemm(self, name, x, k, w, epi, rows, st, **kw):
         a = self.gemm_args(name, x, k, w, epi, **kw)
         a.rows_padded = rows
@@ -752,7 +766,7 @@ class Qwen3TreeEngine(TreeEngineBase):
         emb, emb_layout, emb_sb = self._embedding()
         slot = {li: i for i, li in enumerate(self.layer_ids)}
         hid_parts = []
-        seg = self.PREFILL_SEGMENT
+        seg = self._prefill_segment(len(toks))
         for s0 in range(0, len(toks), seg):
             part = toks[s0:s0 + seg]
             n = len(part)

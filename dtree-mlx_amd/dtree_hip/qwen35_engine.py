@@ -316,7 +316,7 @@ class Qwen35TreeEngine(TreeEngineBase):
         emb, emb_layout, emb_sb = self._embedding()
         slot = {li: i for i, li in enumerate(self.layer_ids)}
         hid_parts = []
-        seg = self.PREFILL_SEGMENT
+        seg = self._prefill_segment(len(toks))
         kv = cache.kv
         for s0 in range(0, len(toks), seg):
             part = toks[s0:s0 + seg]

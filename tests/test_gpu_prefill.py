@@ -250,6 +250,41 @@ def test_prefill_long_matches_oracle(gpu_device, attn_kernel, T, segment, head):
     assert np.abs(lg - last_logits).max() <= TOL * np.abs(last_logits).max()
 
 
+def _short_of_memory(monkeypatch, eng, most):
+    """Allocations of more than `most` prefill rows fail; the rows asked for."""
+    asked, orig = [], eng._prefill_buffers
+
+    def buffers(rows):
+        asked.append(rows)
+        if rows > most:
+            raise torch.cuda.OutOfMemoryError("no room")
+        return orig(rows)
+
+    monkeypatch.setattr(eng, "_prefill_buffers", buffers)
+    return asked
+
+
+def test_prefill_long_takes_smaller_segments_without_memory(gpu_device, monkeypatch):
+    cfg = tiny_qwen3()
+    w = Qwen3Weights.random(cfg, seed=0, device=gpu_device, norm_jitter=0.1)
+    toks = random_prefix(2100, cfg.vocab_size, seed=7)
+    outs = []
+    for most, want in ((4096, [2176, 2176]), (2000, [2176, 2048, 1024] + 3 * [1024])):
+        eng = Qwen3TreeModel(cfg, w, max_past=2200, layer_ids=[1]).engine
+        asked = _short_of_memory(monkeypatch, eng, most)
+        cache = eng.new_cache()
+        logits, hidden = eng.prefill_long(cache, toks)
+        torch.cuda.synchronize()
+        assert asked == want and cache.offset == 2100
+        outs.append((logits.float().cpu().numpy()[0], hidden.float().cpu().numpy()))
+    for (a, b), what in zip(zip(*outs), ("logits", "verifier hidden")):
+        _check_rows(a, b, what)
+    eng = Qwen3TreeModel(cfg, w, max_past=2200, layer_ids=[1]).engine
+    _short_of_memory(monkeypatch, eng, 512)
+    with pytest.raises(torch.cuda.OutOfMemoryError):
+        eng.prefill_long(eng.new_cache(), toks)
+
+
 def test_prefill_long_q4_matches_oracle(gpu_device):
     """The long-M prefill with q4 group-64 weights (every linear layer and the
     tied embedding) against the oracle on the dequantised weights."""
