@@ -8,7 +8,11 @@ rows, and in every output layout an `out` buffer that holds NaN before the call
 
 Bound: the recurrence is a contraction here (|k| = 1, beta and g in [0, 1]), so
 fp32 rounding of a few operations per token adds up to some 2^-24 sqrt(tokens)
-of the result; 2e-6 leaves a factor of ten over what was measured (2e-7)."""
+of the result; 2e-6 leaves a factor of ten over what was measured (2e-7).
+test_chain_keeps_digits holds the sums themselves to account: y's error lies with
+the dot products of 128 dims that A and U are made of (four sums 1.4e-7, one
+chain 2.0e-7), the state's with what is rounded at the state's magnitude (a
+chunk's update at once 2.3e-7, token by token within the chunk 3.6e-7)."""
 import ctypes as C
 
 import pytest
@@ -19,7 +23,8 @@ from dtree_hip import _native as N
 pytestmark = pytest.mark.gpu
 
 
-def _chain(dev, T, Hk=16, Hv=32, kind="random", rowmajor=False, h16=False, stale=False):
+def _chain(dev, T, Hk=16, Hv=32, kind="random", rowmajor=False, h16=False, stale=False,
+           y_tol=2e-6, state_tol=2e-6):
     g = torch.Generator(device=dev)
     g.manual_seed(T + Hk + 7 * Hv + len(kind))
     D = 128
@@ -35,6 +40,8 @@ def _chain(dev, T, Hk=16, Hv=32, kind="random", rowmajor=False, h16=False, stale
         proj[:T, :key * 2] = proj[0, :key * 2]
         proj[:T, Cd + val:Cd + val + Hv] = 8.0          # beta ~ 1
         dt_bias = torch.full((Hv,), -12.0, device=dev)  # g ~ 1
+    elif kind == "slow":  # a state that decays over thousands of tokens
+        dt_bias = torch.full((Hv,), -9.0, device=dev)
     elif kind == "forget":  # g underflows to 0 for some tokens and heads
         proj[:T, Cd + val + Hv:width] *= 60.0
     win, st = rnd(3, Cd), 0.1 * rnd(Hv, D, D)
@@ -75,8 +82,9 @@ def _chain(dev, T, Hk=16, Hv=32, kind="random", rowmajor=False, h16=False, stale
         y[t] = (S @ q[t].unsqueeze(-1)).squeeze(-1)
     got = b["y"][:T].double().reshape(T, Hv, D)
     assert torch.isfinite(got).all()
-    assert ((got - y).norm() / y.norm()).item() <= 2e-6
-    assert ((state.double() - S).norm() / S.norm()).item() <= 2e-6
+    ey, es = ((got - y).norm() / y.norm()).item(), ((state.double() - S).norm() / S.norm()).item()
+    print(f"y {ey:.2e} state {es:.2e}", flush=True)
+    assert ey <= y_tol and es <= state_tol
     assert torch.equal(window, torch.cat([win, proj[:T, :Cd]])[-3:])
     # the gated norm has replaced every scratch value in `out`
     zg = proj[:T, Cd:Cd + val].double().reshape(T, Hv, D)
@@ -118,3 +126,8 @@ def test_chain_row_major_unpadded(gpu_device, T):
 @pytest.mark.parametrize("T", [40, 41, 63, 65, 81, 300])
 def test_chain_ignores_old_out(gpu_device, T, layout):
     _chain(gpu_device, T, 4, 8, rowmajor=layout == "rowmajor", h16=layout == "tiled_f16", stale=True)
+
+
+@pytest.mark.parametrize("kind,T,y_tol,state_tol", [("random", 300, 1.75e-7, 1.4e-7), ("slow", 1024, 3.3e-7, 3e-7)])
+def test_chain_keeps_digits(gpu_device, kind, T, y_tol, state_tol):
+    _chain(gpu_device, T, 4, 8, kind=kind, y_tol=y_tol, state_tol=state_tol)
