@@ -20,8 +20,9 @@
 //   same lane and the row's sum of squares one lane exchange away.
 // * Narrow outputs (fewer tiles than CUs) run eight waves on a 128 x 128 tile,
 //   two groups of four on the two halves of every K block: two waves per SIMD
-//   cover each other's waits (N 2560, K 9728, 1024 rows: 79 us with four
-//   waves, 65 with eight).
+//   cover each other's waits (N 2560, K 9728, 1024 rows, repeated by itself: 79
+//   us with four waves, 65 with eight; as the down projection of a prompt, behind
+//   gate/up, 89).
 //
 // Bound by MFMA issue on the wide tiles (a 256 x 256 tile with no loads at all
 // takes 85 % of its time; the card's clock falls to about 2 GHz under it) and by
@@ -424,12 +425,13 @@ __global__ __launch_bounds__(T::THREADS) void long_kernel(LongParams p) {
 //
 // Measured against the kernel this one replaced (128 x 128 tiles through
 // registers, both folds as FMAs, sum(x) by MFMA in every wave): the 9B-shaped
-// MLP (gate/up and down) over 300 tokens 477 -> 238 us; N 24576, K 4096, 4096
-// rows 846 us (0.98 PFLOP/s; the fp16 tiles reach 1.18). Bound by a wave's own
+// MLP (gate/up and down) over 300 tokens 477 -> 240 us; N 24576, K 4096, 4096
+// rows 847 us (0.97 PFLOP/s; the fp16 tiles reach 1.18). Bound by a wave's own
 // instruction chain (folds, unpacking, load issue, waits): a lone wave per SIMD
 // takes as long per stage as two, and deeper pipelines change nothing. With the
 // folds beginning under their block's last MFMA and the load resources remade
-// from vector registers at every load it was 248 us and 913 us.
+// from vector registers at every load it was 248 us and 913 us (with 128 + q,
+// then 236 and 827).
 constexpr int kRing = 8;        // groups per correction step
 constexpr int kRingStride = 12; // floats per ring row (16-byte reads, spread over the banks)
 
@@ -767,12 +769,12 @@ using T256x256 = Tile<4, 2, 2, 4, 4>;
 using T256x320 = Tile<2, 5, 4, 2, 4>;
 using T256x384 = Tile<4, 3, 2, 4, 3>;
 
-// Tile shape for fp16 operands. One workgroup runs per CU, so a launch takes
-// ceil(tiles / CUs) rounds of one tile time each; the shape with the least
-// rounds x tile time wins. `cost` is the tile time in us per 64 K with every
-// CU busy (a CU's share of the load bandwidth bounds the narrow tiles, MFMA
+// Tile shape for fp16 operands. A launch is taken as ceil(tiles / CUs) rounds of
+// one tile time each (a CU's LDS holds one workgroup, but two of the 64 x 64
+// tiles, which is in their cost); the shape with the least rounds x tile time
+// wins. `cost` is the tile time in us per 64 K with every CU busy (a CU's share of the load bandwidth bounds the narrow tiles, MFMA
 // issue the wide ones; per output element 256 x 256 is the cheapest). Measured
-// for 1024 rows, us (128x128 / 256x128 / 256x192 / 256x256 / 256x320 /
+// for 1024 rows, us, each product repeated by itself (128x128 / 256x128 / 256x192 / 256x256 / 256x320 /
 // 256x384): N 2560 K 9728 65 / 110 / 160 / 179 / 238 / 306; N 6144 K 2560
 // 48 / 42 / 53 / 61 / 70 / 85; N 12352 K 2560 102 / 89 / 112 / 77 / 81 / 103;
 // N 19456 K 2560 136 / 129 / 120 / 133 / 98 / 108; N 24576 K 4096 244 / 212 /
@@ -786,7 +788,8 @@ enum { kT64x64, kT64x128, kT128x128, kT256x128, kT256x192, kT256x256, kT256x320,
 constexpr TileCost kTileCost[kTiles] = {{64, 64, 0.25f}, {64, 128, 0.35f}, {128, 128, 0.55f}, {256, 128, 0.75f},
                                         {256, 192, 1.08f}, {256, 256, 1.30f}, {256, 320, 1.62f}, {256, 384, 2.05f}};
 // The same for q4 weights (one or two K blocks per stage; 128 x 128 tiles need
-// an even number of them). us at 1024 rows (128x128 / 128x256 / 256x192 /
+// an even number of them). Measured with nibbles as 128 + q, 1 to 2 % below the
+// present times, us at 1024 rows (128x128 / 128x256 / 256x192 /
 // 256x256): N 2560 K 9728 106 / 179 / 237 / 286; N 12352 K 2560 136 / 111 / 143
 // / 88; N 24576 K 4096 290 / 256 / 231 / 261; 4096 rows, N 24576 K 4096: 1141
 // / 1021 / 920 / 846; N 2560 K 9728: 316 / 369 / 259 / 289.
