@@ -1682,7 +1682,7 @@ __global__ __launch_bounds__(256) void gdn_chain_scan_kernel(GdnParams p, const 
 }
 
 // ---- the chain in matrix form, 32 tokens at a time ------------------------------
-// (More than 40 tokens; the scan above for fewer.) Unrolled over a chunk of 32 tokens from its first state S_0 (the tree's matrix
+// (More than 40 or 55 tokens; the scan above for fewer.) Unrolled over a chunk of 32 tokens from its first state S_0 (the tree's matrix
 // form with parent t - 1), the recurrence is
 //   Delta = A (V - diag(gamma) K S_0^T),   A = (I + L)^-1 diag(beta),
 //   Y = diag(gamma) Q S_0^T + U Delta,     S_1 = gamma_31 S_0 + (diag(suf) Delta)^T K,
@@ -2469,9 +2469,14 @@ extern "C" int dtree_gdn_layer_chain(const DtreeGdnArgs* a, int32_t num_tokens, 
   p.T = num_tokens; p.Hk = a->num_k_heads; p.Hv = a->num_v_heads; p.Dv = a->head_v_dim; p.y = a->y;
   const int state_blocks = a->num_v_heads * (a->head_v_dim / 8);
   const int conv_blocks = (C + 255) / 256;
-  // Token by token up to 40 tokens (32: 31 us the layer's core, in matrix form 34;
-  // 64: 45 and 35; 1024: 421 and 129).
-  if (num_tokens <= 40) {
+  // Token by token up to 40 tokens where the scan puts more than one workgroup on
+  // a CU, and up to 55 where it does not or a wave of the chunk matrices has more
+  // than one value head to do. The layer's core, us, token by token / in matrix
+  // form: 16 key and 32 value heads, 32 tokens 25.7 / 28, 48 tokens 31.7 / 29.3,
+  // 64 tokens 38 / 31; 8 and 16 heads, 48 tokens 26.0 / 27.7, 56 tokens 28.4 / 27.6;
+  // 4 and 32 heads, 48 tokens 31.0 / 34.2, 56 tokens 34.4 / 34.4.
+  const int scan_tokens = state_blocks > 256 && a->num_v_heads / a->num_k_heads <= 4 ? 40 : 55;
+  if (num_tokens <= scan_tokens) {
     gdn_chain_scan_kernel<<<state_blocks + conv_blocks, 256, 0, stream>>>(p, a->proj, a->ld_proj, a->window, C,
                                                                            a->conv_keep, state_blocks);
     DTREE_LAUNCH_CHECK("gdn_layer_chain scan launch");

@@ -106,6 +106,12 @@ def test_chain_forms(gpu_device, T):
     _chain(gpu_device, T)
 
 
+@pytest.mark.parametrize("Hk,Hv", [(8, 16), (4, 32)])
+@pytest.mark.parametrize("T", [55, 56])
+def test_chain_forms_of_few_heads(gpu_device, T, Hk, Hv):
+    _chain(gpu_device, T, Hk, Hv)
+
+
 @pytest.mark.parametrize("kind", ["repeat", "forget"])
 @pytest.mark.parametrize("T", [50, 200])
 def test_chain_hard_inputs(gpu_device, T, kind):
@@ -117,13 +123,13 @@ def test_chain_head_groups(gpu_device, Hk, Hv):
     _chain(gpu_device, 77, Hk, Hv)
 
 
-@pytest.mark.parametrize("T", [41, 64, 65, 81])
+@pytest.mark.parametrize("T", [41, 56, 64, 65, 81])
 def test_chain_row_major_unpadded(gpu_device, T):
     _chain(gpu_device, T, 2, 4, rowmajor=True)
 
 
 @pytest.mark.parametrize("layout", ["tiled", "tiled_f16", "rowmajor"])
-@pytest.mark.parametrize("T", [40, 41, 63, 65, 81, 300])
+@pytest.mark.parametrize("T", [40, 41, 56, 63, 65, 81, 300])
 def test_chain_ignores_old_out(gpu_device, T, layout):
     _chain(gpu_device, T, 4, 8, rowmajor=layout == "rowmajor", h16=layout == "tiled_f16", stale=True)
 
