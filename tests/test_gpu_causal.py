@@ -107,7 +107,19 @@ def _case(dev, geo, Hq, Hkv, past, n, tiled=True, norms=True, workspace=None, pa
     assert err <= 2e-4, err
     if workspace is not None:
         assert torch.isnan(ws[workspace[0] // 4:]).all()
-        return 1 - torch.isnan(ws).double().mean().item()
+        used = 1 - torch.isnan(ws).double().mean().item()
+        # captured, with eager work between the replays and stale buffers each time
+        first, graph = out.clone(), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            N.check(N.lib().dtree_causal_attention_split(C.byref(a), past, n, ws.data_ptr() + workspace[1], workspace[0],
+                                                         torch.cuda.current_stream().cuda_stream), "causal attention")
+        for _ in range(3):
+            out.fill_(float("nan"))
+            ws.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, first)
+        return used
 
 
 # partial results of one key range: per workgroup (four 32-row units), O and two statistics
